@@ -107,80 +107,71 @@ __device__ __forceinline__ uint32_t decode_pair_h2(uint32_t c0, uint32_t c1, con
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Hand-scheduled gfx950 decode primitives for the GEMV's hot loop.  A 32-bit funnel window `x` holds one codeword
-// in its low half and (for rates K = 1, 2, 4) the codeword 16/K positions earlier in its high half; HI selects it.
-// Every op here is full rate: the 32-bit hash multiply c*M (a quarter-rate v_mul_lo_u32) becomes
-//   t = lo16(c * hi16(M)) << 16        v_mul_lo_u16 (SDWA: reads the 16-bit half, writes the high half)
-//   p = c * lo16(M) + t                v_mad_u32_u16 (op_sel picks the half)
-// which equals c*M mod 2^32 because c < 2^16.
-
-template <bool HI>
-__device__ __forceinline__ uint32_t mul16x32(uint32_t x, uint32_t mh, uint32_t ml) {
-    uint32_t t, p;
-    if constexpr (HI) {
-        asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0"
-            : "=v"(t) : "v"(x), "v"(mh));
-        asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(p) : "v"(x), "v"(ml), "v"(t));
-    } else {
-        asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0"
-            : "=v"(t) : "v"(x), "v"(mh));
-        asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(p) : "v"(x), "v"(ml), "v"(t));
-    }
-    return p;
-}
-
-// The hash products of the GEMV hot loop as two full-rate steps, so a tile's codewords can run each step as one
-// batch (no instruction then reads the result of the one just before it, and the hazard recognizer inserts no wait
-// states):
-//   MCG / hash rows: step 1  t = lo16(c * hi16(M)) << 16       v_mul_lo_u16 (SDWA, high half written, low cleared)
-//                    step 2  t = c * lo16(M) + t               v_mad_u32_u16, in place     -> c*M mod 2^32
-//   3INST (LCG):     step 1  p = c * lo16(A) + B               v_mad_u32_u16
-//                    step 2  p.hi = lo16(c * hi16(A) + p.hi)   v_mad_u16 op_sel (high half written, low kept)
-//                                                              -> c*A + B mod 2^32
+// Hand-scheduled gfx950 decode primitives for the GEMV's and GEMMs' hot loops.  What an instruction costs a SIMD with
+// four waves on it (cycles per wave64 instruction, independent destinations, the slowest wave timed): VGPR-only VOP1 /
+// VOP2 (and, add, shift, f16 add) 2.3-2.5 and v_bitop3 2.7, but 4.2 for the same with one SGPR operand; SDWA and the
+// other VOP3 (alignbit, bfe, mad_u32_u16, perm, packed) 4.2-4.4; v_mul_lo_u32 4.27, no more than its 16-bit parts;
+// v_mad_u16 with op_sel 8.3.  So the hash is one 32-bit product of the clean codeword (and / shift 2.4 + 4.27, where
+// two 16-bit steps took 8.5, 12.6 for the LCG), and every constant a step reads per weight sits in a VGPR.
 constexpr uint32_t LCG_A = 89226354u, LCG_B = 64248484u;
 
-template <int FAM>
-__device__ __forceinline__ uint32_t hash_mult(const DecodeK &k) {
-    return FAM == FAM_MCG ? 0xCBAC1FEDu : FAM == FAM_3INST ? LCG_A : k.mult;
+// s in a VGPR that stays one: written in asm, so the compiler neither folds a scalar operand back in nor rebuilds the
+// constant, and hoists the move out of the loop that uses it.
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t s) {
+    uint32_t v;
+    asm("v_mov_b32 %0, %1" : "=v"(v) : "s"(s));
+    return v;
 }
 
-template <int FAM, bool HI>
-__device__ __forceinline__ uint32_t hash_step1(uint32_t x, const DecodeK &k) {
-    const uint32_t m = hash_mult<FAM>(k);
+// The constants of one decode in VGPRs: multiplier, the masks of the product's halves, the xor (MCG, 3INST) or second
+// mask (PAIR), the LCG's increment, the codeword mask and width.
+struct DecodeV {
+    uint32_t mult, mask, flip, add, wmask, width;
+};
+
+template <int FAM>
+__device__ __forceinline__ DecodeV decode_vgprs(const DecodeK &k) {
+    DecodeV v{};
+    v.mult = in_vgpr(FAM == FAM_MCG ? 0xCBAC1FEDu : FAM == FAM_3INST ? LCG_A : k.mult);
+    v.mask = in_vgpr((FAM == FAM_MCG || FAM == FAM_3INST) ? 0x8FFF8FFFu : k.mask0);
+    if constexpr (FAM == FAM_MCG || FAM == FAM_3INST) v.flip = in_vgpr(0x3B603B60u);
+    else if constexpr (FAM == FAM_PAIR) v.flip = in_vgpr(k.mask1);
+    if constexpr (FAM == FAM_3INST) v.add = in_vgpr(LCG_B);
+    v.wmask = in_vgpr(k.wmask);
+    v.width = 32u - (uint32_t)__builtin_clz(k.wmask);
+    return v;
+}
+
+// c * M mod 2^32 (+ B for the LCG) for a clean codeword c.
+template <int FAM>
+__device__ __forceinline__ uint32_t hash_product(uint32_t c, const DecodeV &v) {
     uint32_t p;
-    if constexpr (FAM == FAM_3INST) {
-        if constexpr (HI)
-            asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(p) : "v"(x), "v"(m & 0xFFFFu), "v"(LCG_B));
-        else
-            asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(p) : "v"(x), "v"(m & 0xFFFFu), "v"(LCG_B));
-    } else {
-        if constexpr (HI)
-            asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0"
-                : "=v"(p) : "v"(x), "v"(m >> 16));
-        else
-            asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_0"
-                : "=v"(p) : "v"(x), "v"(m >> 16));
-    }
+    asm("v_mul_lo_u32 %0, %1, %2" : "=v"(p) : "v"(c), "v"(v.mult));
     return p;
 }
-
-template <int FAM, bool HI>
-__device__ __forceinline__ void hash_step2(uint32_t x, const DecodeK &k, uint32_t &p) {
-    const uint32_t m = hash_mult<FAM>(k);
-    if constexpr (FAM == FAM_3INST) {
-        if constexpr (HI) asm("v_mad_u16 %0, %1, %2, %0 op_sel:[1,0,1,1]" : "+v"(p) : "v"(x), "v"(m >> 16));
-        else asm("v_mad_u16 %0, %1, %2, %0 op_sel:[0,0,1,1]" : "+v"(p) : "v"(x), "v"(m >> 16));
-    } else {
-        if constexpr (HI) asm("v_mad_u32_u16 %0, %1, %2, %0 op_sel:[1,0,0,0]" : "+v"(p) : "v"(x), "v"(m & 0xFFFFu));
-        else asm("v_mad_u32_u16 %0, %1, %2, %0" : "+v"(p) : "v"(x), "v"(m & 0xFFFFu));
-    }
+template <int FAM>
+__device__ __forceinline__ uint32_t hash_add(uint32_t p, const DecodeV &v) {
+    if constexpr (FAM == FAM_3INST) asm("v_add_u32 %0, %0, %1" : "+v"(p) : "v"(v.add));
+    return p;
 }
 
 // The masked product: the f16 pair whose sum is the weight (unscaled for hash rows).
 template <int FAM>
-__device__ __forceinline__ uint32_t hash_halves(uint32_t p, const DecodeK &k) {
-    if constexpr (FAM == FAM_HASH) return p & k.mask0;
-    else return (p & 0x8FFF8FFFu) ^ 0x3B603B60u;
+__device__ __forceinline__ uint32_t hash_halves(uint32_t p, const DecodeV &v) {
+    uint32_t h;
+    if constexpr (FAM == FAM_HASH) asm("v_and_b32 %0, %1, %2" : "=v"(h) : "v"(v.mask), "v"(p));
+    else asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x6a" : "=v"(h) : "v"(p), "v"(v.mask), "v"(v.flip));  // (p & mask) ^ flip
+    return h;
+}
+
+// A weight from its masked product's halves, into the low half of w (the high half cleared) or into the high half.
+__device__ __forceinline__ void half_sum_low(uint32_t &w, uint32_t h) {
+    asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
+        : "=v"(w) : "v"(h));
+}
+__device__ __forceinline__ void half_sum_high(uint32_t &w, uint32_t h) {
+    asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
+        : "+v"(w) : "v"(h));
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -253,6 +244,35 @@ __device__ __forceinline__ uint32_t lane_codeword(const uint32_t (&A)[LaneBits<N
     const int sh = 32 * (a + 1) - e;       // bits of word a after the window
     if (a == 0) return A[0] >> sh;
     return __builtin_amdgcn_alignbit(A[a - 1], A[a], sh);
+}
+
+// Codeword u clean (masked to the window, high bits clear), straight from the words: one bit-field extract (or a mask or
+// a shift) where the 16 bits lie in one word, else a funnel and a mask.
+template <int N, bool MASKED>
+__device__ __forceinline__ uint32_t lane_codeword_clean(const uint32_t (&A)[LaneBits<N>::AW], int u, const DecodeV &v) {
+    const int e = LaneBits<N>::end_of(u), a = (e - 1) >> 5, sh = 32 * (a + 1) - e;
+    uint32_t c;
+    if (sh == 0 || sh > 16) {
+        const uint32_t x = sh == 0 ? A[a] : lane_codeword<N>(A, u);
+        asm("v_and_b32 %0, %1, %2" : "=v"(c) : "v"(v.wmask), "v"(x));
+    } else if (!MASKED && sh == 16) {
+        c = A[a] >> 16;
+    } else {
+        c = __builtin_amdgcn_ubfe(A[a], (uint32_t)sh, MASKED ? v.width : 16u);
+    }
+    return c;
+}
+
+// The codewords of a 32-bit window (Pairing): its low half, and the one its high half holds.
+template <bool MASKED, bool HI>
+__device__ __forceinline__ uint32_t window_codeword(uint32_t x, const DecodeV &v) {
+    if constexpr (!HI) {
+        uint32_t c;
+        asm("v_and_b32 %0, %1, %2" : "=v"(c) : "v"(v.wmask), "v"(x));
+        return c;
+    } else {
+        return MASKED ? __builtin_amdgcn_ubfe(x, 16u, v.width) : x >> 16;
+    }
 }
 
 // Codeword t of a tile at a runtime rate n: the 16 stream bits ending at floor((t+1)n/16), circular

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * RL_WAVES) void reconstruct_tiled_kernel(const 
     uint32_t A[3];
     load_lane_words_tiled(reinterpret_cast<const uint32_t *>(trellis) + seg_off[seg], lw, j, k1, A);
     uint32_t w[16];
-    decode_weights_tiled<FAM, MASKED>(A, k1, tiled_constants(k1, ka, kb), w);
+    decode_weights_tiled<FAM, MASKED>(A, k1, ka, kb, w);
     if constexpr (family_scaled<FAM>()) {
 #pragma unroll
         for (int i = 0; i < 16; i++) w[i] = scale_h2_4096(w[i]);

@@ -419,9 +419,8 @@ struct TiledReader {
     __device__ __forceinline__ void decode(const uint32_t (&W)[AW], uint32_t (&w)[16]) const {
         const uint32_t A[3] = {W[0], W[1], W[2]};
         const bool k1 = W[3] != 0;
-        const DecodeK kl = tiled_constants(k1, ka, kb);
-        if (kb.wmask != 0xFFFFu) decode_weights_tiled<FAM, true>(A, k1, kl, w);
-        else decode_weights_tiled<FAM, false>(A, k1, kl, w);
+        if (kb.wmask != 0xFFFFu) decode_weights_tiled<FAM, true>(A, k1, ka, kb, w);
+        else decode_weights_tiled<FAM, false>(A, k1, ka, kb, w);
     }
 };
 

@@ -175,14 +175,14 @@ __device__ __forceinline__ void decode_tile(const uint32_t (&A)[LaneBits<N>::AW]
     mfma_dot<RT>(w, xs, kk, rows, accA, accB, i4, f0);
 }
 
-// The same for a lane of a per-tile-rate bank, at its own tile's rate (k: the lane's constants).
+// The same for a lane of a per-tile-rate bank, at its own tile's rate (ka / kb: the constants at n = 16 / 32).
 template <int FAM, int RT, bool MASKED>
 __device__ __forceinline__ void decode_tile_tiled(const uint32_t (&A)[3], bool k1, const uint16_t (*xs)[XS_PITCH],
-                                                  int kk, int rows, const DecodeK &k, f4_t (&accA)[RowGroups<RT>::G],
+                                                  int kk, int rows, const DecodeK &ka, const DecodeK &kb, f4_t (&accA)[RowGroups<RT>::G],
                                                   f4_t (&accB)[RowGroups<RT>::G], int i4) {
     const XFrag f0 = read_xfrag(xs, min(i4, RT - 1), kk);
     uint32_t w[16];
-    decode_weights_tiled<FAM, MASKED>(A, k1, k, w);
+    decode_weights_tiled<FAM, MASKED>(A, k1, ka, kb, w);
     mfma_dot<RT>(w, xs, kk, rows, accA, accB, i4, f0);
 }
 
@@ -590,9 +590,10 @@ __device__ __forceinline__ void gemv_body(const GemvArgs &a, GemvCtx &c, const u
         auto decode_at = [&](int t, int tt) __attribute__((always_inline)) {  // slot t holds the wave's tile tt
             const int kk = wave + GEMV_WAVES * tt;
             if constexpr (TILED) {
-                const DecodeK kl = tiled_constants(k1s[t], ts.ka, ts.kb);
-                if (masked) decode_tile_tiled<FAM, RT, true>(Aw[t], k1s[t], xs, kk, c.rows, kl, accA, accB, lane & 3);
-                else decode_tile_tiled<FAM, RT, false>(Aw[t], k1s[t], xs, kk, c.rows, kl, accA, accB, lane & 3);
+                if (masked)
+                    decode_tile_tiled<FAM, RT, true>(Aw[t], k1s[t], xs, kk, c.rows, ts.ka, ts.kb, accA, accB, lane & 3);
+                else
+                    decode_tile_tiled<FAM, RT, false>(Aw[t], k1s[t], xs, kk, c.rows, ts.ka, ts.kb, accA, accB, lane & 3);
             } else {
                 if (masked) decode_tile<FAM, N, RT, true>(Aw[t], xs, kk, c.rows, k, accA, accB, lane & 3);
                 else decode_tile<FAM, N, RT, false>(Aw[t], xs, kk, c.rows, k, accA, accB, lane & 3);

@@ -6,6 +6,8 @@
 #pragma once
 #include "exl3_common.cuh"
 
+#include <type_traits>
+
 namespace exl3 {
 
 // Codeword v of the lane as (window index, high half?): for K = 1, 2, 4 the window ending at codeword v + 16/K
@@ -16,6 +18,7 @@ struct Pairing {
     static constexpr int STEP = ON ? 256 / N : 32;
     __device__ static constexpr bool hi(int v) { return ON && ((v / STEP) % 2 == 0); }
     __device__ static constexpr int win(int v) { return hi(v) ? v + STEP : v; }
+    static constexpr int win_of(int v) { return ON && (v / STEP) % 2 == 0 ? v + STEP : v; }  // on host and device
 };
 
 // A scheduling fence: nothing moves across it, so each phase below stays one batch of independent instructions.
@@ -29,15 +32,97 @@ __device__ __forceinline__ uint32_t scale_h2_4096(uint32_t v) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
+// f(std::integral_constant<int, 0>) .. f(std::integral_constant<int, N - 1>): an unrolled loop whose index is a constant
+// to the code it runs.
+template <int N, class F>
+__device__ __forceinline__ void unrolled(F f) {
+    if constexpr (N > 0) {
+        unrolled<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+// The clean codewords cw(0) .. cw(C - 1) of a lane into c (CW: a constexpr map), in two fenced phases for the paired
+// rates: the windows that hold them, then their halves.
+template <int N, int C, bool MASKED, class CW>
+__device__ __forceinline__ void lane_codewords(const uint32_t (&A)[LaneBits<N>::AW], const DecodeV &v, uint32_t (&c)[C],
+                                               CW) {
+    using P = Pairing<N>;
+    if constexpr (P::ON) {
+        uint32_t win[32];
+        unrolled<C>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int u = CW::at(decltype(ic)::value);
+            if constexpr (CW::first(decltype(ic)::value, P::win(u))) win[P::win(u)] = lane_codeword<N>(A, P::win(u));
+        });
+        phase_fence();
+        unrolled<C>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, u = CW::at(i);
+            c[i] = window_codeword<MASKED, P::hi(u)>(win[P::win(u)], v);
+        });
+    } else {
+        unrolled<C>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            c[i] = lane_codeword_clean<N, MASKED>(A, CW::at(i), v);
+        });
+    }
+    phase_fence();
+}
+
+// Products, masks and sums of C clean codewords (consecutive ones a weight pair) into C / 2 packed pairs, in fenced
+// phases: within a phase no instruction depends on another, so no result is read by the instruction right after it and
+// the hazard recognizer inserts no wait states (gfx950 needs one between an SDWA write and its reader, and counts none
+// for writes in asm).
+template <int FAM, int C>
+__device__ __forceinline__ void hash_weights(uint32_t (&c)[C], const DecodeV &v, uint32_t (&w)[C / 2]) {
+#pragma unroll
+    for (int i = 0; i < C; i++) c[i] = hash_product<FAM>(c[i], v);
+    phase_fence();
+    if constexpr (FAM == FAM_3INST) {
+#pragma unroll
+        for (int i = 0; i < C; i++) c[i] = hash_add<FAM>(c[i], v);
+        phase_fence();
+    }
+#pragma unroll
+    for (int i = 0; i < C; i++) c[i] = hash_halves<FAM>(c[i], v);
+    phase_fence();
+#pragma unroll
+    for (int i = 0; i < C; i += 2) half_sum_low(w[i / 2], c[i]);
+    phase_fence();
+#pragma unroll
+    for (int i = 0; i < C; i += 2) half_sum_high(w[i / 2], c[i + 1]);
+    phase_fence();
+}
+
+// Codeword orders.  `first(i, w)`: no earlier position's window is w.
+template <int N, int C, class At>
+struct CodewordOrder {
+    static constexpr int at(int i) { return At::at(i); }
+    static constexpr bool first(int i, int win) {
+        for (int q = 0; q < i; q++)
+            if (Pairing<N>::win_of(At::at(q)) == win) return false;
+        return true;
+    }
+};
+struct OrderAll {  // all 32 in order
+    static constexpr int at(int i) { return i; }
+};
+template <int N, int G>
+struct OrderGroup {  // group G of two, 16 codewords whose windows hold no other group's (8 apart for n = 16)
+    static constexpr int at(int i) { return N == 16 ? (i < 8 ? 8 * G + i : 8 + 8 * G + i) : 16 * G + i; }
+};
+template <int H, int G>
+struct OrderHalf {  // group G of two of the half decode: column j + 8 H, 8 codewords
+    static constexpr int at(int i) { return 2 * (2 * H + ((i >> 1) & 1) + 4 * (2 * G + (i >> 2))) + (i & 1); }
+};
+
 // The weights of the lane's chunk, unscaled for the hash / pair families (the x4096 is applied by the caller).
-// Written in fenced phases (windows, product step 1, step 2, masks, low sums, high sums): within a phase no
-// instruction depends on another, so no result is read by the instruction right after it and the hazard recognizer
-// inserts no wait states (gfx950 needs one between a 16-bit-lane or SDWA write and its reader).
-template <int FAM, int N, bool MASKED>
+// GROUPED: the phases over two groups of 16 codewords, half the temporaries (a caller whose accumulators need the
+// registers); the others run all 32 together where the rate pairs its windows.
+template <int FAM, int N, bool MASKED, bool GROUPED = !Pairing<N>::ON>
 __device__ __forceinline__ void decode_weights(const uint32_t (&A)[LaneBits<N>::AW], const DecodeK &k,
                                                uint32_t (&w)[16]) {
     using P = Pairing<N>;
-    if constexpr (FAM == FAM_PAIR || FAM == FAM_MUL1) {
+    if constexpr (FAM == FAM_MUL1) {
         uint32_t win[32];
 #pragma unroll
         for (int v = 0; v < 32; v++) {
@@ -46,87 +131,55 @@ __device__ __forceinline__ void decode_weights(const uint32_t (&A)[LaneBits<N>::
                 if constexpr (MASKED) win[v] &= k.wmask | (k.wmask << 16);
             }
         }
-        if constexpr (FAM == FAM_PAIR) {
-            // both weights of a pair decode from the odd codeword (decodePair, expert_exl3.zig:298-301)
-            uint32_t pr[16];
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int v = 2 * i + 1;
-                pr[i] = P::hi(v) ? mul16x32<true>(win[P::win(v)], k.mult >> 16, k.mult & 0xFFFFu)
-                                 : mul16x32<false>(win[P::win(v)], k.mult >> 16, k.mult & 0xFFFFu);
-            }
-            uint32_t h0[16], h1[16];
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                h0[i] = pr[i] & k.mask0;
-                h1[i] = __builtin_amdgcn_alignbit(pr[i], pr[i], 32u - k.rot) & k.mask1;
-            }
-            // the sums in two fenced phases, as the hash-product families write theirs below: each is an SDWA write
-            // in inline asm, whose readers need wait states the compiler does not count for asm (an MFMA reading
-            // one two instructions later read stale weights); phased, a sum is read no sooner than the next phase
-            phase_fence();
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-                    : "=v"(w[i]) : "v"(h0[i]));
-            phase_fence();
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-                    : "+v"(w[i]) : "v"(h1[i]));
-            phase_fence();
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const uint32_t x0 = win[P::win(2 * i)], x1 = win[P::win(2 * i + 1)];
-                const uint32_t c0 = P::hi(2 * i) ? x0 >> 16 : x0, c1 = P::hi(2 * i + 1) ? x1 >> 16 : x1;
-                w[i] = pack_h2(decode1<FAM_MUL1>(c0, k), decode1<FAM_MUL1>(c1, k));
-            }
+        for (int i = 0; i < 16; i++) {
+            const uint32_t x0 = win[P::win(2 * i)], x1 = win[P::win(2 * i + 1)];
+            const uint32_t c0 = P::hi(2 * i) ? x0 >> 16 : x0, c1 = P::hi(2 * i + 1) ? x1 >> 16 : x1;
+            w[i] = pack_h2(decode1<FAM_MUL1>(c0, k), decode1<FAM_MUL1>(c1, k));
         }
+    } else if constexpr (FAM == FAM_PAIR) {
+        const DecodeV v = decode_vgprs<FAM>(k);
+        // both weights of a pair decode from the odd codeword (decodePair, expert_exl3.zig:298-301)
+        uint32_t pr[16];
+        unrolled<16>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            pr[i] = lane_codeword_clean<N, MASKED>(A, 2 * i + 1, v);
+        });
+        phase_fence();
+#pragma unroll
+        for (int i = 0; i < 16; i++) pr[i] = hash_product<FAM>(pr[i], v);
+        phase_fence();
+        uint32_t h0[16], h1[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            h0[i] = pr[i] & v.mask;
+            h1[i] = __builtin_amdgcn_alignbit(pr[i], pr[i], 32u - k.rot) & v.flip;
+        }
+        phase_fence();
+#pragma unroll
+        for (int i = 0; i < 16; i++) half_sum_low(w[i], h0[i]);
+        phase_fence();
+#pragma unroll
+        for (int i = 0; i < 16; i++) half_sum_high(w[i], h1[i]);
+        phase_fence();
     } else {
-        // Rates without pairing (one window per codeword) run the phases over two halves of the chunk, so only half
-        // the windows and products are live at once; paired windows serve codewords up to 16 apart, so paired rates
-        // run all 32 together.
-        constexpr int H = P::ON ? 1 : 2;
-        constexpr int V = 32 / H;
-#pragma unroll
-        for (int hh = 0; hh < H; hh++) {
-            const int v0 = hh * V;
-            uint32_t win[V], h[V];
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                if (P::win(v0 + v) == v0 + v) {
-                    win[v] = lane_codeword<N>(A, v0 + v);
-                    if constexpr (MASKED) win[v] &= k.wmask | (k.wmask << 16);
-                }
-            }
-            phase_fence();
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                const int wv = P::win(v0 + v) - v0;
-                h[v] = P::hi(v0 + v) ? hash_step1<FAM, true>(win[wv], k) : hash_step1<FAM, false>(win[wv], k);
-            }
-            phase_fence();
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                const int wv = P::win(v0 + v) - v0;
-                if (P::hi(v0 + v)) hash_step2<FAM, true>(win[wv], k, h[v]);
-                else hash_step2<FAM, false>(win[wv], k, h[v]);
-            }
-            phase_fence();
-#pragma unroll
-            for (int v = 0; v < V; v++) h[v] = hash_halves<FAM>(h[v], k);
-            phase_fence();
-#pragma unroll
-            for (int i = 0; i < V / 2; i++)
-                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-                    : "=v"(w[v0 / 2 + i]) : "v"(h[2 * i]));
-            phase_fence();
-#pragma unroll
-            for (int i = 0; i < V / 2; i++)
-                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-                    : "+v"(w[v0 / 2 + i]) : "v"(h[2 * i + 1]));
-            phase_fence();
+        const DecodeV v = decode_vgprs<FAM>(k);
+        if constexpr (!GROUPED) {
+            uint32_t c[32];
+            lane_codewords<N, 32, MASKED>(A, v, c, CodewordOrder<N, 32, OrderAll>{});
+            hash_weights<FAM, 32>(c, v, w);
+        } else {
+            unrolled<2>([&](auto gc) __attribute__((always_inline)) {
+                constexpr int g = decltype(gc)::value;
+                using O = OrderGroup<N, g>;
+                uint32_t c[16], p[8];
+                lane_codewords<N, 16, MASKED>(A, v, c, CodewordOrder<N, 16, O>{});
+                hash_weights<FAM, 16>(c, v, p);
+                unrolled<8>([&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    w[O::at(2 * i) / 2] = p[i];
+                });
+            });
         }
     }
 }
@@ -139,42 +192,19 @@ template <int FAM, int N, bool MASKED, int H>
 __device__ __forceinline__ void decode_weights_half(const uint32_t (&A)[LaneBits<N>::AW], const DecodeK &k,
                                                     uint32_t (&w)[8]) {
     static_assert(FAM != FAM_PAIR && FAM != FAM_MUL1, "the half decoder serves the hash-product families");
-    using P = Pairing<N>;
-    // codeword u (0..15) of this half: pair 2H + (u >> 1 & 1) + 4 (u >> 2), element u & 1
-    auto cw_of = [](int u) constexpr { return 2 * (2 * H + ((u >> 1) & 1) + 4 * (u >> 2)) + (u & 1); };
-#pragma unroll
-    for (int gq = 0; gq < 2; gq++) {
-        uint32_t win[8], h[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            win[i] = lane_codeword<N>(A, P::win(cw_of(8 * gq + i)));
-            if constexpr (MASKED) win[i] &= k.wmask | (k.wmask << 16);
-        }
+    const DecodeV v = decode_vgprs<FAM>(k);
+    unrolled<2>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = decltype(gc)::value;
+        uint32_t c[8], p[4];
+        unrolled<8>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            c[i] = lane_codeword_clean<N, MASKED>(A, OrderHalf<H, g>::at(i), v);
+        });
         phase_fence();
+        hash_weights<FAM, 8>(c, v, p);
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            h[i] = P::hi(cw_of(8 * gq + i)) ? hash_step1<FAM, true>(win[i], k) : hash_step1<FAM, false>(win[i], k);
-        phase_fence();
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (P::hi(cw_of(8 * gq + i))) hash_step2<FAM, true>(win[i], k, h[i]);
-            else hash_step2<FAM, false>(win[i], k, h[i]);
-        }
-        phase_fence();
-#pragma unroll
-        for (int i = 0; i < 8; i++) h[i] = hash_halves<FAM>(h[i], k);
-        phase_fence();
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-                : "=v"(w[4 * gq + q]) : "v"(h[2 * q]));
-        phase_fence();
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-                : "+v"(w[4 * gq + q]) : "v"(h[2 * q + 1]));
-        phase_fence();
-    }
+        for (int q = 0; q < 4; q++) w[4 * g + q] = p[q];
+    });
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -206,53 +236,33 @@ __device__ __forceinline__ void load_lane_words_tiled(const uint32_t *__restrict
 // and 16 + s (s >= 8) carry s and 8 + s), so only the window extraction depends on the rate; the products, masks and
 // sums run once over 16 windows in the n = 32 arrangement (codewords 0-7 = high halves 0-7, 8-15 = low 0-7, 16-23 =
 // high 8-15, 24-31 = low 8-15).  At n = 16 the middle two groups of that arrangement hold codewords 16-23 and 8-15,
-// so a k1 lane swaps pairs 4-7 with 8-11 at the end.  k: the lane's rate constants.
+// so a k1 lane swaps pairs 4-7 with 8-11 at the end.  ka / kb: the constants at n = 16 / 32.
 template <int FAM, bool MASKED>
-__device__ __forceinline__ void decode_weights_tiled(const uint32_t (&A)[3], bool k1, const DecodeK &k,
-                                                     uint32_t (&w)[16]) {
+__device__ __forceinline__ void decode_weights_tiled(const uint32_t (&A)[3], bool k1, const DecodeK &ka,
+                                                     const DecodeK &kb, uint32_t (&w)[16]) {
     static_assert(FAM != FAM_PAIR && FAM != FAM_MUL1, "per-tile rates serve the hash-product families");
     const uint32_t A16[2] = {A[0], A[1]};
-    uint32_t win[16], hl[16], hh[16];
+    DecodeV v = decode_vgprs<FAM>(kb);
+    if constexpr (FAM == FAM_HASH) {  // the rows differ by rate: the lane's own
+        v.mult = k1 ? in_vgpr(ka.mult) : v.mult;
+        v.mask = k1 ? in_vgpr(ka.mask0) : v.mask;
+    }
+    uint32_t win[16], c[32];
 #pragma unroll
     for (int s = 0; s < 16; s++) {
         const uint32_t c16 = lane_codeword<16>(A16, 16 + s);
         const uint32_t c32 = lane_codeword<32>(A, s < 8 ? 8 + s : 16 + s);
         win[s] = k1 ? c16 : c32;
-        if constexpr (MASKED) win[s] &= k.wmask | (k.wmask << 16);
     }
     phase_fence();
+    // codeword u of the n = 32 arrangement
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-        hl[s] = hash_step1<FAM, false>(win[s], k);
-        hh[s] = hash_step1<FAM, true>(win[s], k);
+    for (int u = 0; u < 32; u++) {
+        const uint32_t x = win[u < 8 ? u : u < 16 ? u - 8 : u < 24 ? u - 8 : u - 16];
+        c[u] = (u & 8) ? window_codeword<MASKED, false>(x, v) : window_codeword<MASKED, true>(x, v);
     }
     phase_fence();
-#pragma unroll
-    for (int s = 0; s < 16; s++) {
-        hash_step2<FAM, false>(win[s], k, hl[s]);
-        hash_step2<FAM, true>(win[s], k, hh[s]);
-    }
-    phase_fence();
-#pragma unroll
-    for (int s = 0; s < 16; s++) {
-        hl[s] = hash_halves<FAM>(hl[s], k);
-        hh[s] = hash_halves<FAM>(hh[s], k);
-    }
-    phase_fence();
-    // codeword v of the n = 32 arrangement
-    auto h_of = [&](int v) __attribute__((always_inline)) {
-        return v < 8 ? hh[v] : v < 16 ? hl[v - 8] : v < 24 ? hh[v - 8] : hl[v - 16];
-    };
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-            : "=v"(w[i]) : "v"(h_of(2 * i)));
-    phase_fence();
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-            : "+v"(w[i]) : "v"(h_of(2 * i + 1)));
-    phase_fence();
+    hash_weights<FAM, 32>(c, v, w);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const uint32_t a = w[4 + q], b = w[8 + q];
@@ -266,15 +276,6 @@ __device__ __forceinline__ void decode_weights_tiled(const uint32_t (&A)[3], boo
 __device__ __forceinline__ uint32_t seg_mask(const uint8_t *k1, size_t seg) {
     const uint32_t w = reinterpret_cast<const uint32_t *>(k1)[seg >> 2];
     return (w >> (8u * (uint32_t)(seg & 3))) & 0xFFu;
-}
-
-// A lane's rate constants in a per-tile-rate bank: the hash rows differ by rate (mult, mask); the window mask and the
-// fixed families' constants do not.
-__device__ __forceinline__ DecodeK tiled_constants(bool k1, const DecodeK &ka, const DecodeK &kb) {
-    DecodeK k = kb;
-    k.mult = k1 ? ka.mult : kb.mult;
-    k.mask0 = k1 ? ka.mask0 : kb.mask0;
-    return k;
 }
 
 }  // namespace exl3
