@@ -13,6 +13,8 @@
 // walked back by one lane per tile.  Codeword values are decoded on the fly (decode1), bit-exact with the engine's.
 #include "exl3_kernels.h"
 
+#include <type_traits>
+
 // The f64 squared error is summed term by term as the reference does; no multiply-add contraction in this file
 // (the path costs' fused multiply-add is written out as fmaf).
 #pragma clang fp contract(off)
@@ -84,6 +86,59 @@ __device__ __forceinline__ void search_step(int step, int ri, int n, int w, cons
             curr[t * 2 * stride + e] = f32_to_f16_bits(best[t]);
             row[t * back_tile + e] = (uint8_t)bf[t];
         }
+    }
+}
+
+// A workgroup's paths to its outputs: packed codes, and where asked the squared error and the decoded values.
+template <int FAM>
+__device__ __forceinline__ void write_outputs(int T, int n, const DecodeK &dk, int64_t tile0, int64_t count,
+                                              const uint16_t *path, uint32_t *words, const float *xs,
+                                              uint16_t *__restrict__ packed, double *__restrict__ sse,
+                                              float *__restrict__ recon) {
+    const int tid = threadIdx.x;
+    // packStates: step t's fresh k bits (the state's low bits), MSB first, end at bitEnd(t) of a stream read as
+    // 32-bit words whose bit 31 comes first; stored little-endian, a word is the halfword pair (lo, hi).
+    for (int i = tid; i < T * 64; i += ENC_THREADS) words[i] = 0u;
+    __syncthreads();
+    for (int i = tid; i < T * 256; i += ENC_THREADS) {
+        const int t = i >> 8, s = i & 255;
+        const int k = fresh_bits(n, s);
+        const int end = ((s + 1) * n) >> 4;
+        const uint32_t field = (uint32_t)path[i] & ((1u << k) - 1u);
+        const int p0 = end - k;
+        const int j0 = p0 >> 5, o0 = p0 & 31;
+        if (o0 + k <= 32) {
+            atomicOr(&words[t * 64 + j0], field << (32 - o0 - k));
+        } else {
+            const int hi = 32 - o0;  // bits in the first word
+            atomicOr(&words[t * 64 + j0], field >> (k - hi));
+            atomicOr(&words[t * 64 + j0 + 1], field << (32 - (k - hi)));
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < T * (n / 2); i += ENC_THREADS) {
+        const int t = i / (n / 2), j = i % (n / 2);
+        if (tile0 + t < count) {
+            const uint32_t v = words[t * 64 + j];
+            packed[(tile0 + t) * n + 2 * j] = (uint16_t)(v & 0xFFFFu);
+            packed[(tile0 + t) * n + 2 * j + 1] = (uint16_t)(v >> 16);
+        }
+    }
+    // The values the decoder will produce, back in row-major tile order.
+    if (recon != nullptr)
+        for (int i = tid; i < T * 256; i += ENC_THREADS) {
+            const int t = i >> 8, j = i & 255;
+            if (tile0 + t < count)
+                recon[(tile0 + t) * 256 + tensor_core_perm(j)] = __half2float(decode1<FAM>(path[i], dk));
+        }
+    // The path's squared error in f64, summed in trellis order as the reference does.
+    if (sse != nullptr && tid < T && tile0 + tid < count) {
+        double acc = 0.0;
+        for (int i = 0; i < 256; i++) {
+            const double d = (double)xs[tid * 256 + i] - (double)__half2float(decode1<FAM>(path[tid * 256 + i], dk));
+            acc += d * d;
+        }
+        sse[tile0 + tid] = acc;
     }
 }
 
@@ -175,51 +230,250 @@ __global__ __launch_bounds__(ENC_THREADS) void encode_search_kernel(const float 
             }
             __syncthreads();
         }
-        // packStates: step t's fresh k bits (the state's low bits), MSB first, end at bitEnd(t) of a stream read as
-        // 32-bit words whose bit 31 comes first; stored little-endian, a word is the halfword pair (lo, hi).
-        for (int i = tid; i < T * 64; i += ENC_THREADS) words[i] = 0u;
+        write_outputs<FAM>(T, n, dk, tile0, count, path, words, xs, packed, sse, recon);
         __syncthreads();
+    }
+}
+
+// The uniform search, for rates whose steps all take the same K = 2, 3 or 4 fresh bits (n = 32, 48, 64).
+//
+// Bound: the VALU.  Every step scores the same codewords, and the 2^K edges of a group (e >> K equal) share the 2^K
+// predecessors fresh << (kr - K) | e >> K.  So a thread owns B blocks of NE consecutive edges of a group for the whole
+// search: their NE x 2^K values are decoded once, into VGPRs, a predecessor's cost is read and widened once for NE
+// edges, and what is left per score is a subtract, a multiply-add and the selection (the general kernel's 9.1
+// lane-instructions per score, decode and per-score cost read among them; 6.2 here, 3.6 in the steps without
+// backpointers).  4096 tiles at n = 32, w = 12, MCG: 2.86 -> 1.19 ms.  Where the blocks are fewer than the
+// threads, the threads split into sets that take the tiles in turn.  Only the steps that a traceback walks keep
+// backpointers: the first half of pass 0 takes minima alone.
+//
+// A block's backpointers are one NE * K-bit word (8 or 12 bits for NE = 4), so a step's row is a quarter to half of
+// one byte an edge.  The traceback reads rows in chunks that half a wave copies to LDS (the cost rows are dead by
+// then), the next chunk in flight while one lane walks this one: a lane that followed the chain through memory waited
+// its latency 384 times.
+//
+// Step 0 has no predecessor: pass 0 starts from zero costs, pass 1 from zero at the pinned edge and 65504 elsewhere,
+// whose scores never beat the starting 65504 (as the reference's: no such edge has a backpointer or a lower cost).
+template <int NE, int K>
+using BackWord = typename std::conditional<(NE * K > 8), uint16_t, uint8_t>::type;
+
+constexpr int CHUNK_BYTES = 2048;  // a tile's backpointer rows copied to LDS at a time: 64 bytes a lane
+
+template <int NE, int K, int B, bool BACK>
+__device__ __forceinline__ void uniform_step(const float (&v)[B][1 << K][NE], const float *xs, int ri, int T, int set,
+                                             int sets, int block, const uint16_t *prev, uint16_t *curr, int stride,
+                                             int pstep, BackWord<NE, K> *row, size_t back_tile) {
+    constexpr int KK = 1 << K;
+    for (int t = set; t < T; t += sets) {
+        const float target = xs[t * 256 + ri];
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            const int blk = block + b * ENC_THREADS;
+            const uint16_t *pc = prev + (size_t)t * 2 * stride + ((blk * NE) >> K);
+            float best[NE];
+            uint32_t bf[NE];
+#pragma unroll
+            for (int f = 0; f < KK; f++) {
+                const float pcost = f16_bits_to_f32(pc[f * pstep]);
+#pragma unroll
+                for (int j = 0; j < NE; j++) {
+                    const float dh = v[b][f][j] - target;
+                    const float err = __builtin_fmaf(dh, dh, pcost);
+                    if (f == 0) {
+                        best[j] = __builtin_fminf(H_INF, err);
+                        bf[j] = 0;
+                    } else {
+                        if (BACK) bf[j] = err < best[j] ? (uint32_t)f : bf[j];
+                        best[j] = __builtin_fminf(best[j], err);
+                    }
+                }
+            }
+            uint16_t h[NE];
+            uint32_t bits = 0;
+#pragma unroll
+            for (int j = 0; j < NE; j++) {
+                h[j] = f32_to_f16_bits(best[j]);
+                bits |= bf[j] << (K * j);
+            }
+            __builtin_memcpy(__builtin_assume_aligned(curr + (size_t)t * 2 * stride + blk * NE, NE * 2), h, NE * 2);
+            if (BACK) row[(size_t)t * back_tile + blk] = (BackWord<NE, K>)bits;
+        }
+    }
+}
+
+template <int FAM, int NE, int K, int B>
+__global__ __launch_bounds__(ENC_THREADS) void encode_uniform_kernel(const float *__restrict__ tiles, int64_t count,
+                                                                     int T, int w, DecodeK dk,
+                                                                     uint16_t *__restrict__ packed,
+                                                                     double *__restrict__ sse,
+                                                                     float *__restrict__ recon,
+                                                                     uint8_t *__restrict__ back_ws) {
+    using Word = BackWord<NE, K>;
+    constexpr int KK = 1 << K;
+    extern __shared__ __align__(16) unsigned char enc_lds[];
+    const int kr = w - K, stride = 1 << kr, blocks = stride / NE;
+    // The general kernel's LDS layout.
+    uint16_t *costs = reinterpret_cast<uint16_t *>(enc_lds);
+    float *xs = reinterpret_cast<float *>(enc_lds + (size_t)T * 2 * stride * 2);
+    uint16_t *path = reinterpret_cast<uint16_t *>(xs + T * 256);
+    uint32_t *words = reinterpret_cast<uint32_t *>(path + T * 256);
+    uint32_t *red = words + T * 64;
+    int *pin = reinterpret_cast<int *>(red + (ENC_THREADS / 64) * T);
+
+    const size_t back_tile = (size_t)256 * blocks;  // Words
+    Word *back = reinterpret_cast<Word *>(back_ws + (size_t)blockIdx.x * T * 256 * stride);
+    const int64_t batches = (count + T - 1) / T;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int block = B == 1 ? tid & (blocks - 1) : tid;
+    const int set = B == 1 ? tid / blocks : 0, sets = B == 1 ? ENC_THREADS / blocks : 1;
+    const int pstep = 1 << (kr - K);
+
+    float v[B][KK][NE];
+#pragma unroll
+    for (int b = 0; b < B; b++)
+#pragma unroll
+        for (int f = 0; f < KK; f++)
+#pragma unroll
+            for (int j = 0; j < NE; j++)
+                v[b][f][j] = __half2float(
+                    decode1<FAM>(((uint32_t)f << kr) | (uint32_t)((block + b * ENC_THREADS) * NE + j), dk));
+
+    // Traceback geometry: half a wave per tile (T <= 16), rows of blocks * sizeof(Word) bytes, chunks of `rows` rows
+    // that fit the tile's cost rows.
+    const int ht = tid >> 5, hl = tid & 31;
+    const int row_bytes = blocks * (int)sizeof(Word);
+    const int chunk = 4 * stride < CHUNK_BYTES ? 4 * stride : CHUNK_BYTES;
+    // Rows wider than a chunk are walked in place.
+    const int rows = row_bytes <= chunk ? chunk / row_bytes : 0;
+
+    for (int64_t bt = blockIdx.x; bt < batches; bt += gridDim.x) {
+        const int64_t tile0 = bt * T;
         for (int i = tid; i < T * 256; i += ENC_THREADS) {
-            const int t = i >> 8, s = i & 255;
-            const int k = fresh_bits(n, s);
-            const int end = ((s + 1) * n) >> 4;
-            const uint32_t field = (uint32_t)path[i] & ((1u << k) - 1u);
-            const int p0 = end - k;
-            const int j0 = p0 >> 5, o0 = p0 & 31;
-            if (o0 + k <= 32) {
-                atomicOr(&words[t * 64 + j0], field << (32 - o0 - k));
-            } else {
-                const int hi = 32 - o0;  // bits in the first word
-                atomicOr(&words[t * 64 + j0], field >> (k - hi));
-                atomicOr(&words[t * 64 + j0 + 1], field << (32 - (k - hi)));
-            }
+            const int t = i >> 8, j = i & 255;
+            const int64_t tile = tile0 + t < count ? tile0 + t : count - 1;
+            xs[i] = tiles[tile * 256 + tensor_core_perm(j)];
         }
+        for (int pass = 0; pass < 2; pass++) {
+            const int roll = pass == 0 ? 128 : 0;
+            for (int i = tid; i < T << kr; i += ENC_THREADS) {
+                const int t = i >> kr, e = i & (stride - 1);
+                costs[t * 2 * stride + e] = pass == 0 || e == pin[t] ? 0 : 0x7BFF;
+            }
+            __syncthreads();
+            for (int step = 0; step < 256; step++) {
+                const int ri = (step + roll) & 255;
+                const uint16_t *prev = costs + (step & 1) * stride;
+                uint16_t *curr = costs + ((step & 1) ^ 1) * stride;
+                Word *row = back + (size_t)ri * blocks;
+                if (pass == 0 && step < 128)
+                    uniform_step<NE, K, B, false>(v, xs, ri, T, set, sets, block, prev, curr, stride, pstep, row,
+                                                  back_tile);
+                else
+                    uniform_step<NE, K, B, true>(v, xs, ri, T, set, sets, block, prev, curr, stride, pstep, row,
+                                                 back_tile);
+                __syncthreads();
+            }
+            if (pass == 0) {  // the first cheapest final edge (256 steps: the last costs are in row 0)
+                for (int t = 0; t < T; t++) {
+                    uint32_t key = 0xFFFFFFFFu;
+                    for (int e = tid; e < stride; e += ENC_THREADS) {
+                        const uint32_t kv = ((uint32_t)costs[t * 2 * stride + e] << 16) | (uint32_t)e;
+                        key = kv < key ? kv : key;
+                    }
+                    for (int off = 32; off > 0; off >>= 1) {
+                        const uint32_t o = (uint32_t)__shfl_xor((int)key, off);
+                        key = o < key ? o : key;
+                    }
+                    if (lane == 0) red[wave * T + t] = key;
+                }
+                __syncthreads();
+                if (tid < T) {
+                    uint32_t key = 0xFFFFFFFFu;
+                    for (int u = 0; u < ENC_THREADS / 64; u++) key = red[u * T + tid] < key ? red[u * T + tid] : key;
+                    pin[tid] = (int)(key & 0xFFFFu);
+                }
+                __syncthreads();
+            }
+            // Traceback of trellis steps 127 .. 0 (pass 0) or 255 .. 0 (pass 1), whose rows lie in order of ri.
+            if (ht < T) {
+                const Word *src = back + (size_t)ht * back_tile;
+                const int top = pass == 0 ? 128 : 256;
+                int edge = pin[ht];
+                auto walk = [&](const Word *r, int ri) {
+                    const int fresh = ((uint32_t)r[edge / NE] >> (K * (edge & (NE - 1)))) & (KK - 1);
+                    const int state = (fresh << kr) | edge;
+                    edge = state >> K;
+                    if (pass == 1) path[ht * 256 + ri] = (uint16_t)state;
+                };
+                if (rows != 0) {
+                    unsigned char *stage = enc_lds + (size_t)ht * 4 * stride;
+                    const unsigned char *bytes = reinterpret_cast<const unsigned char *>(src);
+                    uint4 q0, q1, q2, q3;  // a chunk's shares of this lane, 512 bytes apart
+                    const bool two = chunk > 512, four = chunk > 1024;
+                    auto fetch = [&](int c) {
+                        const unsigned char *from = bytes + (size_t)c * chunk + hl * 16;
+                        q0 = *reinterpret_cast<const uint4 *>(from);
+                        if (two) q1 = *reinterpret_cast<const uint4 *>(from + 512);
+                        if (four) q2 = *reinterpret_cast<const uint4 *>(from + 1024);
+                        if (four) q3 = *reinterpret_cast<const uint4 *>(from + 1536);
+                    };
+                    const int chunks = top / rows;
+                    fetch(chunks - 1);
+                    for (int c = chunks - 1; c >= 0; c--) {
+                        unsigned char *to = stage + hl * 16;
+                        *reinterpret_cast<uint4 *>(to) = q0;
+                        if (two) *reinterpret_cast<uint4 *>(to + 512) = q1;
+                        if (four) *reinterpret_cast<uint4 *>(to + 1024) = q2;
+                        if (four) *reinterpret_cast<uint4 *>(to + 1536) = q3;
+                        if (c > 0) fetch(c - 1);
+                        // The half wave runs in step: its stores are ordered before its own reads.
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                        for (int r = rows - 1; r >= 0; r--)
+                            walk(reinterpret_cast<const Word *>(stage + r * row_bytes), c * rows + r);
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    }
+                } else {
+                    for (int ri = top - 1; ri >= 0; ri--) walk(src + (size_t)ri * blocks, ri);
+                }
+                if (hl == 0) pin[ht] = edge;
+            }
+            __syncthreads();
+        }
+        write_outputs<FAM>(T, K * 16, dk, tile0, count, path, words, xs, packed, sse, recon);
         __syncthreads();
-        for (int i = tid; i < T * (n / 2); i += ENC_THREADS) {
-            const int t = i / (n / 2), j = i % (n / 2);
-            if (tile0 + t < count) {
-                const uint32_t v = words[t * 64 + j];
-                packed[(tile0 + t) * n + 2 * j] = (uint16_t)(v & 0xFFFFu);
-                packed[(tile0 + t) * n + 2 * j + 1] = (uint16_t)(v >> 16);
-            }
-        }
-        // The values the decoder will produce, back in row-major tile order.
-        if (recon != nullptr)
-            for (int i = tid; i < T * 256; i += ENC_THREADS) {
-                const int t = i >> 8, j = i & 255;
-                if (tile0 + t < count)
-                    recon[(tile0 + t) * 256 + tensor_core_perm(j)] = __half2float(decode1<FAM>(path[i], dk));
-            }
-        // The path's squared error in f64, summed in trellis order as the reference does.
-        if (sse != nullptr && tid < T && tile0 + tid < count) {
-            double acc = 0.0;
-            for (int i = 0; i < 256; i++) {
-                const double d = (double)xs[tid * 256 + i] - (double)__half2float(decode1<FAM>(path[tid * 256 + i], dk));
-                acc += d * d;
-            }
-            sse[tile0 + tid] = acc;
-        }
-        __syncthreads();
+    }
+}
+
+template <int FAM, int NE, int K, int B>
+hipError_t launch_uniform(const EncodeArgs &a, hipStream_t s) {
+    const size_t lds = encode_lds_bytes(a.tiles_per_wg, a.stride);
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&encode_uniform_kernel<FAM, NE, K, B>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((encode_uniform_kernel<FAM, NE, K, B>), dim3((unsigned)a.grid), dim3(ENC_THREADS), lds, s,
+                       a.tiles, a.count, a.tiles_per_wg, a.w, a.k, a.packed, a.sse, a.recon, a.back);
+    return hipGetLastError();
+}
+
+// NE edges a thread: as many as share the predecessors' reads while a thread's values (NE x 2^K x B) stay within 128
+// VGPRs; fewer where one tile a workgroup would leave threads without edges.
+template <int FAM, int K>
+hipError_t launch_uniform_k(const EncodeArgs &a, hipStream_t s) {
+    constexpr int NE = K == 4 ? 2 : 4;
+    if (K < 4 && a.tiles_per_wg == 1 && a.w == 12) return launch_uniform<FAM, K == 2 ? 2 : 1, K, 1>(a, s);
+    switch (a.stride / NE / ENC_THREADS) {
+    case 0:
+    case 1: return launch_uniform<FAM, NE, K, 1>(a, s);
+    case 2: return launch_uniform<FAM, NE, K, 2>(a, s);
+    case 4: return launch_uniform<FAM, NE, K, 4>(a, s);
+    default:  // 8: K = 2 at a 16-bit window
+        if constexpr (K == 2) return launch_uniform<FAM, NE, K, 8>(a, s);
+        return hipErrorInvalidValue;
     }
 }
 
@@ -238,6 +492,12 @@ hipError_t launch_encode(const EncodeArgs &a, hipStream_t s) {
 
 template <int FAM>
 hipError_t launch_encode_t(const EncodeArgs &a, hipStream_t s) {
+    // The uniform search copies backpointer rows by 16 bytes, so it wants an aligned workspace.
+    if (a.w >= 12 && a.w <= 16 && (reinterpret_cast<uintptr_t>(a.back) & 15) == 0) {
+        if (a.n == 32) return launch_uniform_k<FAM, 2>(a, s);
+        if (a.n == 48) return launch_uniform_k<FAM, 3>(a, s);
+        if (a.n == 64) return launch_uniform_k<FAM, 4>(a, s);
+    }
     switch (a.tiles_per_wg) {
     case 16: return launch_encode<FAM, 16>(a, s);
     case 8: return launch_encode<FAM, 8>(a, s);

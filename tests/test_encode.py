@@ -225,3 +225,48 @@ def test_gpu_search_with_a_one_workgroup_workspace_runs_every_batch(dev):
     for i in itertools.islice(range(count), 0, count, 7):
         p, s, _ = O.encode_tile(tiles[i], n, O.decode(O.CB_MCG, w))
         np.testing.assert_array_equal(want[i], p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cb,n,w,count", [
+    (O.CB_MCG, 32, 12, 1), (O.CB_MCG, 32, 12, 600), (O.CB_MUL1, 32, 12, 2051),  # 1, 2 and 8 tiles a workgroup
+    (O.CB_3INST, 32, 13, 1030), (O.CB_MCG, 32, 14, 300), (O.CB_MUL1, 32, 15, 17), (O.CB_MCG, 32, 16, 9),
+    (O.CB_MUL1, 48, 12, 3), (O.CB_MCG, 48, 12, 4099), (O.CB_MCG, 48, 14, 515), (O.CB_3INST, 48, 15, 19),
+    (O.CB_MUL1, 48, 16, 5), (O.CB_MCG, 64, 12, 2), (O.CB_3INST, 64, 12, 4100), (O.CB_MUL1, 64, 13, 1025),
+    (O.CB_MCG, 64, 14, 259), (O.CB_MCG, 64, 15, 18), (O.CB_MUL1, 64, 16, 7)])
+def test_the_uniform_search_is_the_general_search(dev, cb, n, w, count):
+    """n = 32, 48, 64 take the uniform kernel at a 16-byte aligned workspace and the general one otherwise: the same
+    codes and errors from both, tiles of zeros, values past the cost clamp, infinities and NaN among them."""
+    import torch
+
+    from sushi_amd import _lib, exl3
+
+    L = _lib.load()
+    rng = np.random.default_rng(n * 31 + w + count)
+    tiles = (rng.standard_normal((count, 256)) * rng.uniform(0.2, 3.0, (count, 1))).astype(np.float32)
+    plain = np.arange(count) % 11 != 10
+    for i, v in zip(np.flatnonzero(~plain), itertools.cycle((0.0, 300.0, 1e6, np.inf, np.nan))):
+        tiles[i, rng.integers(0, 256, 200)] = v
+    if count > 1:
+        tiles[0] = 0.0
+    t = torch.from_numpy(tiles).to(dev)
+    dec = exl3.Decode(exl3.Codebook(cb), exl3.Window(w))
+    size = L.exl3_encode_workspace_size(n, dec.c(), count)
+    ws = torch.empty(size + 16, dtype=torch.uint8, device=dev)
+    assert ws.data_ptr() % 16 == 0
+    stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    got = []
+    for off in (0, 1):
+        packed = torch.zeros(count, n, dtype=torch.int16, device=dev)
+        sse = torch.zeros(count, dtype=torch.float64, device=dev)
+        rc = L.exl3_encode_tiles(t.data_ptr(), count, n, dec.c(), packed.data_ptr(), sse.data_ptr(),
+                                 ws.data_ptr() + off, size, stream)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        got.append((packed.cpu().numpy().view(np.uint16), sse.cpu().numpy()))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    i = int(np.flatnonzero(plain)[-1])
+    want, want_sse, _ = O.encode_tile(tiles[i], n, O.decode(cb, w))
+    np.testing.assert_array_equal(got[0][0][i], want)
+    assert got[0][1][i] == want_sse
