@@ -182,7 +182,7 @@ uint32_t gemm_split_wait(long workgroups) {
 
 size_t gemm_bytes(int groups, int rows, int in, int out, int n, bool split_ok = true) {
     size_t b = kZeroBytes + gemm_xp_bytes(groups, rows, in);
-    const bool lane_reader = n == 16 || n == 24 || n == 32 || n == 40 || n == 48 || n == 64;
+    const bool lane_reader = lane_rate(n) || n == 80 || n == 96 || n == 112 || n == 128;
     if (!lane_reader) b += align_up((size_t)groups * out * in * 2);  // the transposed f16 copy of other rates
     if (gemm_uses_kpart(groups, rows, out, n, split_ok)) b += align_up(gemm_kpart_bytes(groups, rows, out));
     return b;

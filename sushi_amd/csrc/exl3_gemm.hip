@@ -1294,20 +1294,23 @@ static hipError_t launch_gemm_lane_n(const GemmArgs &a, hipStream_t s) {
     // halves, 224 workgroups, 3% faster).
     int arm = a.arm ? a.arm : gemm_default_arm(a.groups, a.rows, a.out);
     if constexpr (FAM == FAM_PAIR || FAM == FAM_MUL1) arm = 4;  // the ping-pong body serves the hash-product families
+    if constexpr (N > 64) arm = 4;  // K = 5 .. 8 are built for the decode-wave tile only
     // n = 40's unaligned lane reader does not fit the 512-row tile's registers (it would spill): the 256-row one
     if constexpr (N == 40) arm = arm == 5 ? (a.arm ? 6 : 4) : arm;
     if (arm == 7 && (N == 40 || !a.kpart)) arm = 4;  // the split needs its partial region (the host sizes it)
-    if (arm == 5 || arm == 6 || arm == 7) {
-        const int mt = arm == 6 ? 256 : 512;
-        dim3 grid((unsigned)((a.out / 128) * ((a.rows + mt - 1) / mt) * (arm == 7 ? 2 : 1)), 1, (unsigned)a.groups);
-        if constexpr (FAM != FAM_PAIR && FAM != FAM_MUL1) {
-            if constexpr (N != 40) {
-                if (arm == 5) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 512, 1>), grid, dim3(G5_THREADS), 0, s, a);
-                if (arm == 7) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 512, 2>), grid, dim3(G5_THREADS), 0, s, a);
+    if constexpr (N <= 64) {
+        if (arm == 5 || arm == 6 || arm == 7) {
+            const int mt = arm == 6 ? 256 : 512;
+            dim3 grid((unsigned)((a.out / 128) * ((a.rows + mt - 1) / mt) * (arm == 7 ? 2 : 1)), 1, (unsigned)a.groups);
+            if constexpr (FAM != FAM_PAIR && FAM != FAM_MUL1) {
+                if constexpr (N != 40) {
+                    if (arm == 5) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 512, 1>), grid, dim3(G5_THREADS), 0, s, a);
+                    if (arm == 7) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 512, 2>), grid, dim3(G5_THREADS), 0, s, a);
+                }
+                if (arm == 6) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 256, 1>), grid, dim3(G5_THREADS), 0, s, a);
             }
-            if (arm == 6) hipLaunchKernelGGL((gemm5_kernel<FAM, N, 256, 1>), grid, dim3(G5_THREADS), 0, s, a);
+            return hipGetLastError();
         }
-        return hipGetLastError();
     }
     dim3 grid((unsigned)((a.out / 128) * ((a.rows + G2_MT - 1) / G2_MT)), 1, (unsigned)a.groups);
     hipLaunchKernelGGL((gemm4_kernel<FAM, N>), grid, dim3(G4_THREADS), 0, s, a);
@@ -1331,6 +1334,19 @@ static hipError_t launch_gemm_fam(const GemmArgs &a, hipStream_t s) {
     case 48: return launch_gemm_lane_n<FAM, 48>(a, s);
     case 64: return launch_gemm_lane_n<FAM, 64>(a, s);
     default: break;
+    }
+    // K = 5 .. 8 (PAIR1 has no rows there): the lane reader inside the tile, instead of a pass that writes the f16
+    // weights and a body that reads them back.  MCG n = 96, 17 / 200 / 777 / 2048 rows: 2560 x 16384 139 / 169 / 243 /
+    // 481 -> 37 / 53 / 119 / 234 us, 14336 x 4096 429 / 533 / 552 / 637 -> 118 / 189 / 211 / 287 us; MUL1 at 14336 x 4096
+    // 440 / 545 / 561 / 646 -> 192 / 274 / 294 / 366 us.
+    if constexpr (FAM != FAM_PAIR) {
+        switch (a.n) {
+        case 80: return launch_gemm_lane_n<FAM, 80>(a, s);
+        case 96: return launch_gemm_lane_n<FAM, 96>(a, s);
+        case 112: return launch_gemm_lane_n<FAM, 112>(a, s);
+        case 128: return launch_gemm_lane_n<FAM, 128>(a, s);
+        default: break;
+        }
     }
     hipLaunchKernelGGL(gemm_prepare_kernel, dim3((unsigned)(a.in / 128), (unsigned)a.rows, (unsigned)a.groups),
                        dim3(64), 0, s, a);

@@ -37,3 +37,14 @@ def test_moe_wide_rates(dev, n, rows):
     y = exl3.moe_with_shared_bank(x.to(dev), _to(b, dev), _to(sh, dev), torch.from_numpy(inds.view(np.int32)).to(dev),
                                   torch.from_numpy(scores).to(dev), exl3.MCG)
     assert max_abs_rel(y.float().cpu().numpy(), want) < BAR
+
+
+@pytest.mark.parametrize("label", ["mcg", "3inst", "mul1", "spec1"])
+@pytest.mark.parametrize("n,rows", [(80, 17), (80, 300), (96, 40), (96, 257), (112, 130), (112, 16 * 8 + 1), (128, 64),
+                                    (128, 520)])
+def test_gemm_wide_rates(dev, label, n, rows):
+    """The GEMM tile at those rates: one to three row tiles with tails, four and eight decode waves (the switch lies at
+    128 rows), k of three 128-blocks, held as the GEMV is."""
+    d = Dense(dev, 940 + n + rows, rows, 384, 256, n)
+    dec, odec = DECODES[label]
+    _hold(d.inner(dec), d, odec, seed=n + rows, what=f"wide gemm {label} n={n} rows={rows}")
