@@ -1464,6 +1464,9 @@ int32_t encode_plan(int32_t n, const exl3_decode_t &dec, int64_t count, EncodePl
     // A small batch (the quantizer's 16-row groups, the global scale's samples) spreads over the CUs first: fewer
     // tiles per workgroup until there is a workgroup per CU.
     while (p->tiles_per_wg > 1 && (count + p->tiles_per_wg - 1) / p->tiles_per_wg < 256) p->tiles_per_wg >>= 1;
+    // The uniform search shares no decode between tiles, so it goes on to two workgroups a CU, down to two tiles each.
+    if (n == 32 || n == 48 || n == 64)
+        while (p->tiles_per_wg > 2 && (count + p->tiles_per_wg - 1) / p->tiles_per_wg < 512) p->tiles_per_wg >>= 1;
     const size_t lds = encode_lds_bytes(p->tiles_per_wg, p->stride);
     int per_cu = (int)((160 * 1024) / lds);
     per_cu = per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu;

@@ -300,8 +300,9 @@ __device__ __forceinline__ void uniform_step(const float (&v)[B][1 << K][NE], co
     }
 }
 
+// Up to 16 values a thread, two workgroups share a CU (at most 128 VGPRs): one's barriers under the other's steps.
 template <int FAM, int NE, int K, int B>
-__global__ __launch_bounds__(ENC_THREADS) void encode_uniform_kernel(const float *__restrict__ tiles, int64_t count,
+__global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void encode_uniform_kernel(const float *__restrict__ tiles, int64_t count,
                                                                      int T, int w, DecodeK dk,
                                                                      uint16_t *__restrict__ packed,
                                                                      double *__restrict__ sse,
@@ -464,15 +465,15 @@ hipError_t launch_uniform(const EncodeArgs &a, hipStream_t s) {
 // VGPRs; fewer where one tile a workgroup would leave threads without edges.
 template <int FAM, int K>
 hipError_t launch_uniform_k(const EncodeArgs &a, hipStream_t s) {
-    constexpr int NE = K == 4 ? 2 : 4;
+    constexpr int NE = K == 2 ? 4 : 2;
     if (K < 4 && a.tiles_per_wg == 1 && a.w == 12) return launch_uniform<FAM, K == 2 ? 2 : 1, K, 1>(a, s);
     switch (a.stride / NE / ENC_THREADS) {
     case 0:
     case 1: return launch_uniform<FAM, NE, K, 1>(a, s);
     case 2: return launch_uniform<FAM, NE, K, 2>(a, s);
     case 4: return launch_uniform<FAM, NE, K, 4>(a, s);
-    default:  // 8: K = 2 at a 16-bit window
-        if constexpr (K == 2) return launch_uniform<FAM, NE, K, 8>(a, s);
+    default:  // 8: K = 2, 3 at a 16-bit window
+        if constexpr (K < 4) return launch_uniform<FAM, NE, K, 8>(a, s);
         return hipErrorInvalidValue;
     }
 }
