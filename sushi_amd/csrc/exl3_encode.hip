@@ -246,8 +246,8 @@ __global__ __launch_bounds__(ENC_THREADS) void encode_search_kernel(const float 
 // threads, the threads split into sets that take the tiles in turn.  Only the steps that a traceback walks keep
 // backpointers: the first half of pass 0 takes minima alone.
 //
-// A block's backpointers are one NE * K-bit word (8 or 12 bits for NE = 4), so a step's row is a quarter to half of
-// one byte an edge.  The traceback reads rows in chunks that half a wave copies to LDS (the cost rows are dead by
+// A block's backpointers are one word of NE * K bits, a byte at the widths launched here, so a step's row is a quarter
+// to a half byte an edge.  The traceback reads rows in chunks that half a wave copies to LDS (the cost rows are dead by
 // then), the next chunk in flight while one lane walks this one: a lane that followed the chain through memory waited
 // its latency 384 times.
 //
@@ -461,8 +461,9 @@ hipError_t launch_uniform(const EncodeArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// NE edges a thread: as many as share the predecessors' reads while a thread's values (NE x 2^K x B) stay within 128
-// VGPRs; fewer where one tile a workgroup would leave threads without edges.
+// NE edges a thread: four at K = 2, where they are the whole group; two at K = 3 and 4, whose larger groups would take
+// the VGPRs of a second workgroup (K = 3, 4 edges: 150, and 700 tiles 627 us against 407); fewer at 12 bits where one
+// tile a workgroup would leave threads without edges.
 template <int FAM, int K>
 hipError_t launch_uniform_k(const EncodeArgs &a, hipStream_t s) {
     constexpr int NE = K == 2 ? 4 : 2;
