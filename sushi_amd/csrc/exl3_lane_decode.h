@@ -139,29 +139,34 @@ __device__ __forceinline__ void decode_weights(const uint32_t (&A)[LaneBits<N>::
         }
     } else if constexpr (FAM == FAM_PAIR) {
         const DecodeV v = decode_vgprs<FAM>(k);
-        // both weights of a pair decode from the odd codeword (decodePair, expert_exl3.zig:298-301)
-        uint32_t pr[16];
-        unrolled<16>([&](auto ic) __attribute__((always_inline)) {
-            constexpr int i = decltype(ic)::value;
-            pr[i] = lane_codeword_clean<N, MASKED>(A, 2 * i + 1, v);
+        // Both weights of a pair decode from the odd codeword (decodePair, expert_exl3.zig:298-301).  Two groups of eight
+        // pairs: 16 codewords with both their half arrays at once took 82-86 VGPRs in the decode GEMV (67-78 in groups,
+        // but for n = 24 and 40), past the 80 that keep three workgroups on a CU.  Routed + shared layer of 128 experts,
+        // 2048 x 768, 32 tokens, together / in groups: n = 32 121 / 115 us, n = 48 130 / 126 us, n = 64 127 / 122 us.
+        unrolled<2>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            uint32_t h0[8], h1[8];
+            unrolled<8>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                h1[i] = lane_codeword_clean<N, MASKED>(A, 2 * (8 * g + i) + 1, v);
+            });
+            phase_fence();
+#pragma unroll
+            for (int i = 0; i < 8; i++) h1[i] = hash_product<FAM>(h1[i], v);
+            phase_fence();
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                h0[i] = h1[i] & v.mask;
+                h1[i] = __builtin_amdgcn_alignbit(h1[i], h1[i], 32u - k.rot) & v.flip;
+            }
+            phase_fence();
+#pragma unroll
+            for (int i = 0; i < 8; i++) half_sum_low(w[8 * g + i], h0[i]);
+            phase_fence();
+#pragma unroll
+            for (int i = 0; i < 8; i++) half_sum_high(w[8 * g + i], h1[i]);
+            phase_fence();
         });
-        phase_fence();
-#pragma unroll
-        for (int i = 0; i < 16; i++) pr[i] = hash_product<FAM>(pr[i], v);
-        phase_fence();
-        uint32_t h0[16], h1[16];
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            h0[i] = pr[i] & v.mask;
-            h1[i] = __builtin_amdgcn_alignbit(pr[i], pr[i], 32u - k.rot) & v.flip;
-        }
-        phase_fence();
-#pragma unroll
-        for (int i = 0; i < 16; i++) half_sum_low(w[i], h0[i]);
-        phase_fence();
-#pragma unroll
-        for (int i = 0; i < 16; i++) half_sum_high(w[i], h1[i]);
-        phase_fence();
     } else {
         const DecodeV v = decode_vgprs<FAM>(k);
         if constexpr (!GROUPED) {

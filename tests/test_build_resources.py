@@ -1,5 +1,6 @@
-"""Every kernel of the built gfx950 library runs without scratch memory and without VGPR spills, and no matrix
-instruction reads a VGPR that a vector instruction wrote fewer than three instructions before it.
+"""Every kernel of the built gfx950 library runs without scratch memory and without VGPR spills, the PAIR decode GEMV
+keeps the registers of three workgroups a CU, and no matrix instruction reads a VGPR that a vector instruction wrote
+fewer than three instructions before it.
 
 Read from the code-object metadata of the objects `python -m sushi_amd.build` leaves in sushi_amd/_build
 (`.private_segment_fixed_size`, `.vgpr_spill_count`).  Scratch in these kernels has meant the compiler copying a
@@ -43,7 +44,7 @@ def _device_object(obj: str, tmp) -> str:
 
 
 def _kernels(obj: str, tmp) -> list:
-    """(name, private segment bytes, VGPR spills) of every kernel in obj's gfx950 code object."""
+    """(name, private segment bytes, VGPR spills, VGPRs) of every kernel in obj's gfx950 code object."""
     dev = _device_object(obj, tmp)
     notes = subprocess.run([READELF, "--notes", dev], capture_output=True, text=True, check=True).stdout
     out = []
@@ -53,7 +54,7 @@ def _kernels(obj: str, tmp) -> list:
         if name is None:
             continue
         out.append((name.group(1), int(field("private_segment_fixed_size").group(1)),
-                    int(field("vgpr_spill_count").group(1))))
+                    int(field("vgpr_spill_count").group(1)), int(field("vgpr_count").group(1))))
     return out
 
 
@@ -64,8 +65,23 @@ def test_no_kernel_uses_scratch_or_spills(tmp_path):
     # the GEMV, GEMM, MoE, decode and encoder objects all hold kernels (the C-ABI object holds none)
     for name in ("exl3_gemv_3inst.o", "exl3_gemm.o", "exl3_moe.o", "exl3_decode.o", "exl3_encode.o"):
         assert kernels.get(name), f"no kernel metadata read from {name}"
-    bad = [(o, n, scratch, spills) for o, ks in kernels.items() for n, scratch, spills in ks if scratch or spills]
+    bad = [(o, n, scratch, spills) for o, ks in kernels.items() for n, scratch, spills, _ in ks if scratch or spills]
     assert not bad, f"{len(bad)} kernels with scratch bytes / VGPR spills, e.g. {bad[:3]}"
+
+
+@pytest.mark.skipif(not OBJECTS or not (os.path.exists(BUNDLER) and os.path.exists(READELF) and shutil.which("objcopy")),
+                    reason="needs the built objects (python -m sushi_amd.build) and the ROCm binutils")
+def test_pair_gemv_keeps_three_workgroups_a_cu(tmp_path):
+    """PAIR's dense, per-slot and windows kernels of 1, 2 and 4 rows at the paired rates and n = 48: at most 80 VGPRs,
+    six waves a SIMD, which is three of their 512-thread workgroups on a CU (gemv_kernel<FAM_PAIR = 3, N, RT, PRO_X = 0, ..>)."""
+    vgprs = {}
+    for name, _, _, v in _kernels(os.path.join(BUILD, "exl3_gemv_pair.o"), str(tmp_path)):
+        m = re.search(r"gemv_kernelILi3ELi(32|48|64)ELi([124])ELi0ELb[01]ELb[01]E", name)
+        if m:
+            vgprs[name] = v
+    assert len(vgprs) == 18, sorted(vgprs)
+    over = {n: v for n, v in vgprs.items() if v > 80}
+    assert not over, over
 
 
 _VREG = re.compile(r"v\[(\d+):(\d+)\]|\bv(\d+)\b")
