@@ -41,9 +41,14 @@ __device__ __forceinline__ int tensor_core_perm(int i) {
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float v) { return __half_as_ushort(__float2half_rn(v)); }
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 
-// One step of the search for all T tiles: scores every codeword, writes each edge's minimum and backpointer.
-template <int FAM, int T>
-__device__ __forceinline__ void search_step(int step, int ri, int n, int w, const DecodeK &dk, const float *xs,
+// One step of the search for all T tiles: scores every codeword, writes each edge's minimum and backpointer.  The first
+// step, which has no predecessor's cost, is a body of its own (FIRST): with its branch in the scoring loop, a dozen
+// instructions a score, the loop's time hung on where the compiler happened to place it (two builds of the same loop
+// 2 - 8% apart).  MCG, branch in the loop (those two builds) / a body of its own: n = 80 w = 12, 64 tiles 1430 - 1535 /
+// 1175 us, 1024 tiles 4300 - 4350 / 1890 us; n = 40 w = 15, 2048 tiles 13.5 - 13.9 / 10.9 ms; n = 24 w = 16, 256 tiles
+// 7.4 - 7.7 / 6.0 ms.
+template <int FAM, int T, bool FIRST>
+__device__ __forceinline__ void search_step(int ri, int n, int w, const DecodeK &dk, const float *xs,
                                             const uint16_t *prev, uint16_t *curr, uint8_t *back, size_t back_tile,
                                             int stride, bool pinned, const int *pin) {
     const int k = fresh_bits(n, ri);
@@ -68,7 +73,7 @@ __device__ __forceinline__ void search_step(int step, int ri, int n, int w, cons
             for (int t = 0; t < T; t++) {
                 const float dh = v - target[t];
                 float err;
-                if (step == 0) {
+                if constexpr (FIRST) {
                     if (pinned && (int)pred != pin[t]) {
                         err = H_INF;
                     } else {
@@ -178,8 +183,12 @@ __global__ __launch_bounds__(ENC_THREADS) void encode_search_kernel(const float 
             int cur = 0;
             for (int step = 0; step < 256; step++) {
                 const int ri = (step + roll) & 255;
-                search_step<FAM, T>(step, ri, n, w, dk, xs, costs + cur * stride, costs + (cur ^ 1) * stride, back,
-                                    back_tile, stride, pass == 1, pin);
+                const uint16_t *prev = costs + cur * stride;
+                uint16_t *curr = costs + (cur ^ 1) * stride;
+                if (step == 0)
+                    search_step<FAM, T, true>(ri, n, w, dk, xs, prev, curr, back, back_tile, stride, pass == 1, pin);
+                else
+                    search_step<FAM, T, false>(ri, n, w, dk, xs, prev, curr, back, back_tile, stride, pass == 1, pin);
                 cur ^= 1;
                 __syncthreads();
             }
