@@ -11,6 +11,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 
 #include "sushi_exl3_hip.h"
 #include "exl3_kernels.h"
@@ -1437,6 +1438,22 @@ struct EncodePlan {
     size_t per_wg;
 };
 
+// The launch of `tiles` tiles a workgroup: backpointers per workgroup, and a grid of at most the workgroups whose LDS
+// fits the CUs (four a CU).
+void encode_shape(int64_t count, int tiles, EncodePlan *p) {
+    p->tiles_per_wg = tiles;
+    const size_t lds = encode_lds_bytes(tiles, p->stride);
+    int per_cu = (int)((160 * 1024) / lds);
+    per_cu = per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu;
+    const int64_t batches = (count + tiles - 1) / tiles;
+    const int64_t cap = 256LL * per_cu;
+    p->grid_max = (int)(batches < cap ? batches : cap);
+    p->per_wg = (size_t)tiles * 256 * p->stride;
+}
+
+// Tiles a workgroup keeps within about half a CU's 160 KB of LDS (one tile always).
+bool encode_tiles_fit(int tiles, int stride) { return tiles == 1 || encode_lds_bytes(tiles, stride) <= 78 * 1024; }
+
 // Encoder.init (src/encoder/encode.zig:120-160): the searchable codebooks (MCG, MUL1; 3INST as this build's
 // extension), an admitted rate, a window of 12..16 bits wider than every step's fresh bits.
 int32_t encode_plan(int32_t n, const exl3_decode_t &dec, int64_t count, EncodePlan *p) {
@@ -1457,25 +1474,45 @@ int32_t encode_plan(int32_t n, const exl3_decode_t &dec, int64_t count, EncodePl
         return fail(EXL3_ERR_WINDOW_TOO_NARROW, "encode: window %d carries no state at n=%d", dec.window_bits, n);
     p->w = dec.window_bits;
     p->stride = 1 << (p->w - kmin);
-    // Tiles per workgroup: as many as keep the workgroup's LDS within about half a CU's 160 KB.
-    p->tiles_per_wg = 1;
-    for (int t = 16; t >= 2; t >>= 1)
-        if (encode_lds_bytes(t, p->stride) <= 78 * 1024) { p->tiles_per_wg = t; break; }
+    // Tiles per workgroup: as many as fit.
+    int tiles = 16;
+    while (!encode_tiles_fit(tiles, p->stride)) tiles >>= 1;
     // A small batch (the quantizer's 16-row groups, the global scale's samples) spreads over the CUs first: fewer
     // tiles per workgroup until there is a workgroup per CU.
-    while (p->tiles_per_wg > 1 && (count + p->tiles_per_wg - 1) / p->tiles_per_wg < 256) p->tiles_per_wg >>= 1;
-    // The uniform search shares no decode between tiles, so it goes on to two workgroups a CU, down to two tiles each.
+    while (tiles > 1 && (count + tiles - 1) / tiles < 256) tiles >>= 1;
+    // The rates of the uniform search go on to two workgroups a CU, down to two tiles each: it shares no decode between
+    // tiles, and two of its workgroups fit a CU at 2 and 3 bits up to a 14-bit window (at most 128 VGPRs; 3000 tiles
+    // n = 32 w = 12 1189 -> 971 us).  Its other instances: encode_plan_alone.
     if (n == 32 || n == 48 || n == 64)
-        while (p->tiles_per_wg > 2 && (count + p->tiles_per_wg - 1) / p->tiles_per_wg < 512) p->tiles_per_wg >>= 1;
-    const size_t lds = encode_lds_bytes(p->tiles_per_wg, p->stride);
-    int per_cu = (int)((160 * 1024) / lds);
-    per_cu = per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu;
-    const int64_t batches = (count + p->tiles_per_wg - 1) / p->tiles_per_wg;
-    const int64_t cap = 256LL * per_cu;
-    p->grid_max = (int)(batches < cap ? batches : cap);
-    p->per_wg = (size_t)p->tiles_per_wg * 256 * p->stride;
+        while (tiles > 2 && (count + tiles - 1) / tiles < 512) tiles >>= 1;
+    encode_shape(count, tiles, p);
     return ok();
 }
+
+// The uniform search's instances of more than 128 VGPRs (4 bits; 2 and 3 bits at 15 and 16), whose workgroups have a CU
+// each: the count of tiles a workgroup whose rounds over 256 CUs end first.  A workgroup's time is its tiles' scores plus
+// what every step costs whatever its tiles (barriers, the traceback), as much as 6144 scores an eighth of a thread each:
+// n = 64 w = 12 measured 283 / 309 / 418 / 746 / 1356 us at 1 / 2 / 4 / 8 / 16 tiles, w = 15 804 / 1469 / 2698 us at
+// 1 / 2 / 4.  Against the two-a-CU rule, n = 64 w = 12: 300 tiles 586 -> 319 us, 700 630 -> 437, 1024 648 -> 448, 4096
+// 1602 -> 1432; n = 48 w = 16, 700 tiles 5.56 -> 4.46 ms; n = 32 w = 15, 300 tiles 1620 -> 1385 us.  False: not such an
+// instance, and p is left as it is.
+bool encode_plan_alone(int32_t n, int64_t count, EncodePlan *p) {
+    if (n != 64 && !((n == 32 || n == 48) && p->w >= 15)) return false;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int tiles = 1; tiles <= 16 && encode_tiles_fit(tiles, p->stride); tiles <<= 1) {
+        const int64_t rounds = ((count + tiles - 1) / tiles + 255) / 256;
+        const int64_t cost = rounds * (((int64_t)tiles << p->w) + 6144);
+        if (cost < least) {
+            least = cost;
+            best = tiles;
+        }
+    }
+    encode_shape(count, best, p);
+    return true;
+}
+
+size_t encode_plan_bytes(const EncodePlan &p) { return (size_t)p.grid_max * p.per_wg; }
 
 EncodeTuning tuning_of(const EncodePlan &p) { return EncodeTuning{p.stride, p.tiles_per_wg, p.grid_max, p.per_wg}; }
 
@@ -1491,6 +1528,10 @@ int32_t quantize_plan(int32_t in, int32_t out, int32_t n, const exl3_decode_t &d
     if (rc) return rc;
     rc = encode_plan(n, dec, out / 16, &pr);
     if (rc) return rc;
+    for (auto [p, count] : {std::pair<EncodePlan *, int64_t>{&pg, 128}, {&pr, out / 16}}) {
+        EncodePlan alone = *p;
+        if (encode_plan_alone(n, count, &alone) && encode_plan_bytes(alone) <= encode_plan_bytes(*p)) *p = alone;
+    }
     *tg = tuning_of(pg);
     *tr = tuning_of(pr);
     return ok();
@@ -1501,7 +1542,8 @@ int32_t quantize_plan(int32_t in, int32_t out, int32_t n, const exl3_decode_t &d
 size_t exl3_encode_workspace_size(int32_t n, exl3_decode_t dec, int64_t count) {
     EncodePlan p;
     if (encode_plan(n, dec, count, &p) != EXL3_OK) return 0;
-    return (size_t)p.grid_max * p.per_wg;
+    const size_t bytes = encode_plan_bytes(p);
+    return encode_plan_alone(n, count, &p) ? std::max(bytes, encode_plan_bytes(p)) : bytes;
 }
 
 int32_t exl3_encode_tiles(const float *tiles, int64_t count, int32_t n, exl3_decode_t dec, uint16_t *packed,
@@ -1511,10 +1553,17 @@ int32_t exl3_encode_tiles(const float *tiles, int64_t count, int32_t n, exl3_dec
     if (rc) return rc;
     if (count == 0) return ok();
     if (!tiles || !packed) return fail(EXL3_ERR_BAD_SHAPE, "encode: null operand");
-    const size_t fit = workspace ? workspace_bytes / p.per_wg : 0;
+    size_t fit = workspace ? workspace_bytes / p.per_wg : 0;
     if (fit < 1)
         return fail(EXL3_ERR_WORKSPACE, "encode: workspace of %zu bytes holds no search (%zu per workgroup)",
                     workspace_bytes, p.per_wg);
+    // The uniform search runs on an aligned workspace; one that holds less than its whole grid keeps the smaller shape.
+    EncodePlan alone = p;
+    if (reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && encode_plan_alone(n, count, &alone) &&
+        workspace_bytes >= encode_plan_bytes(alone)) {
+        p = alone;
+        fit = p.grid_max;
+    }
     int fam;
     DecodeK k;
     rc = resolve_decode(dec, n, &fam, &k);

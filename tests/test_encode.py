@@ -227,9 +227,35 @@ def test_gpu_search_with_a_one_workgroup_workspace_runs_every_batch(dev):
         np.testing.assert_array_equal(want[i], p)
 
 
+def _plan_tiles(n, w, cb, count):
+    """Tiles a workgroup, read from the workspace query: 256 backpointer rows of 2^(w - k) bytes for the tiles rounded up
+    to whole workgroups, where the count lies one past a multiple of 16 and no grid is capped."""
+    from sushi_amd import _lib, exl3
+
+    size = _lib.load().exl3_encode_workspace_size(n, exl3.Decode(exl3.Codebook(cb), exl3.Window(w)).c(), count)
+    per_tile = 256 << (w - n // 16)
+    assert count % 16 == 1 and size % per_tile == 0
+    return size // per_tile - count + 1
+
+
+# (codebook, n, w, tiles, tiles a workgroup) of the uniform search: every tile count a workgroup it is launched with, a
+# last batch with one live tile in each.  At 2 and 3 bits up to w = 14 two workgroups share a CU (512 of them before a
+# workgroup takes more tiles, at least two); the others have a CU each (the fewest rounds over 256).
+UNIFORM_PLANS = [
+    (O.CB_MCG, 32, 12, 1, 1), (O.CB_MCG, 32, 12, 593, 2), (O.CB_MUL1, 32, 12, 2049, 4), (O.CB_MCG, 32, 12, 4097, 8),
+    (O.CB_3INST, 32, 14, 2033, 2), (O.CB_MCG, 32, 15, 305, 2), (O.CB_MUL1, 48, 12, 4097, 8), (O.CB_MCG, 48, 12, 8177, 16),
+    (O.CB_MCG, 48, 15, 1009, 4), (O.CB_MCG, 64, 12, 305, 2), (O.CB_MUL1, 64, 12, 1009, 4), (O.CB_MCG, 64, 12, 2033, 8),
+    (O.CB_3INST, 64, 12, 4081, 16), (O.CB_MUL1, 64, 13, 1009, 4), (O.CB_MCG, 64, 14, 305, 2)]
+
+
+@pytest.mark.parametrize("cb,n,w,count,tiles", UNIFORM_PLANS)
+def test_the_uniform_search_plan(cb, n, w, count, tiles):
+    assert _plan_tiles(n, w, cb, count) == tiles
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("cb,n,w,count", [
-    (O.CB_MCG, 32, 12, 1), (O.CB_MCG, 32, 12, 600), (O.CB_MUL1, 32, 12, 2051),  # 1, 2 and 8 tiles a workgroup
+@pytest.mark.parametrize("cb,n,w,count", [p[:4] for p in UNIFORM_PLANS] + [
+    (O.CB_MCG, 32, 12, 600), (O.CB_MUL1, 32, 12, 2051), (O.CB_MCG, 32, 12, 4096),
     (O.CB_3INST, 32, 13, 1030), (O.CB_MCG, 32, 14, 300), (O.CB_MUL1, 32, 15, 17), (O.CB_MCG, 32, 16, 9),
     (O.CB_MUL1, 48, 12, 3), (O.CB_MCG, 48, 12, 4099), (O.CB_MCG, 48, 14, 515), (O.CB_3INST, 48, 15, 19),
     (O.CB_MUL1, 48, 16, 5), (O.CB_MCG, 64, 12, 2), (O.CB_3INST, 64, 12, 4100), (O.CB_MUL1, 64, 13, 1025),
@@ -270,3 +296,28 @@ def test_the_uniform_search_is_the_general_search(dev, cb, n, w, count):
     want, want_sse, _ = O.encode_tile(tiles[i], n, O.decode(cb, w))
     np.testing.assert_array_equal(got[0][0][i], want)
     assert got[0][1][i] == want_sse
+
+
+@pytest.mark.gpu
+def test_gpu_search_on_a_short_workspace_at_a_rate_with_a_cu_each(dev):
+    """n = 64 takes four tiles a workgroup at this count; a workspace that holds one workgroup of the two-tile shape (what
+    such a workspace always had to hold) is accepted, runs every batch and gives the same codes."""
+    import torch
+
+    from sushi_amd import _lib, exl3
+
+    L = _lib.load()
+    n, w, count = 64, 12, 1009
+    assert _plan_tiles(n, w, O.CB_MCG, count) == 4
+    tiles = np.random.default_rng(5).standard_normal((count, 256)).astype(np.float32)
+    dec = exl3.Decode(exl3.Codebook.mcg, exl3.Window(w))
+    two = 2 * 256 << (w - 4)
+    t = torch.from_numpy(tiles).to(dev)
+    ws = torch.empty(two, dtype=torch.uint8, device=dev)
+    packed = torch.zeros(count, n, dtype=torch.int16, device=dev)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    args = (t.data_ptr(), count, n, dec.c(), packed.data_ptr(), 0, ws.data_ptr())
+    assert L.exl3_encode_tiles(*args, two - 1, stream) == exl3.Exl3WorkspaceTooSmall.status
+    assert L.exl3_encode_tiles(*args, two, stream) == 0, _lib.last_error()
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(packed.cpu().numpy().view(np.uint16), _gpu_encode(dev, tiles, n, O.CB_MCG, w)[0])
