@@ -13,8 +13,6 @@
 // walked back by one lane per tile.  Codeword values are decoded on the fly (decode1), bit-exact with the engine's.
 #include "exl3_kernels.h"
 
-#include <type_traits>
-
 // The f64 squared error is summed term by term as the reference does; no multiply-add contraction in this file
 // (the path costs' fused multiply-add is written out as fmaf).
 #pragma clang fp contract(off)
@@ -249,28 +247,25 @@ __global__ __launch_bounds__(ENC_THREADS) void encode_search_kernel(const float 
 // Bound: the VALU.  Every step scores the same codewords, and the 2^K edges of a group (e >> K equal) share the 2^K
 // predecessors fresh << (kr - K) | e >> K.  So a thread owns B blocks of NE consecutive edges of a group for the whole
 // search: their NE x 2^K values are decoded once, into VGPRs, a predecessor's cost is read and widened once for NE
-// edges, and what is left per score is a subtract, a multiply-add and the selection (the general kernel's 9.1
-// lane-instructions per score, decode and per-score cost read among them; 6.2 here, 3.6 in the steps without
-// backpointers).  4096 tiles at n = 32, w = 12, MCG: 2.86 -> 1.19 ms.  Where the blocks are fewer than the
-// threads, the threads split into sets that take the tiles in turn.  Only the steps that a traceback walks keep
+// edges, and what is left per score is a subtract, a multiply-add and the selection: with four edges, 6.2 instructions a
+// score in the compiled loop, 3.6 in the steps without backpointers, each score's share of the reads and addresses
+// included.  4096 tiles at n = 32, w = 12, MCG: 2.13 ms by the general search, 1.20 ms here.  Where the blocks are fewer
+// than the threads, the threads split into sets that take the tiles in turn.  Only the steps that a traceback walks keep
 // backpointers: the first half of pass 0 takes minima alone.
 //
-// A block's backpointers are one word of NE * K bits, a byte at the widths launched here, so a step's row is a quarter
-// to a half byte an edge.  The traceback reads rows in chunks that half a wave copies to LDS (the cost rows are dead by
-// then), the next chunk in flight while one lane walks this one: a lane that followed the chain through memory waited
-// its latency 384 times.
+// A block's backpointers, NE * K bits, are a byte: a step's row is a quarter byte an edge (2 bits) or half (3 and 4
+// bits; a half and one with a single tile a workgroup at 12 bits).  The traceback reads rows in chunks that half a wave
+// copies to LDS (the cost rows are dead by then), the next chunk in flight while the half wave walks this one, its lanes
+// in step along the one path: a lane that followed the chain through memory waited its latency 384 times.
 //
 // Step 0 has no predecessor: pass 0 starts from zero costs, pass 1 from zero at the pinned edge and 65504 elsewhere,
 // whose scores never beat the starting 65504 (as the reference's: no such edge has a backpointer or a lower cost).
-template <int NE, int K>
-using BackWord = typename std::conditional<(NE * K > 8), uint16_t, uint8_t>::type;
-
-constexpr int CHUNK_BYTES = 2048;  // a tile's backpointer rows copied to LDS at a time: 64 bytes a lane
+constexpr int CHUNK_BYTES = 2048;  // a tile's backpointer rows copied to LDS at a time: 32 or 64 bytes a lane
 
 template <int NE, int K, int B, bool BACK>
 __device__ __forceinline__ void uniform_step(const float (&v)[B][1 << K][NE], const float *xs, int ri, int T, int set,
                                              int sets, int block, const uint16_t *prev, uint16_t *curr, int stride,
-                                             int pstep, BackWord<NE, K> *row, size_t back_tile) {
+                                             int pstep, uint8_t *row, size_t back_tile) {
     constexpr int KK = 1 << K;
     for (int t = set; t < T; t += sets) {
         const float target = xs[t * 256 + ri];
@@ -304,20 +299,18 @@ __device__ __forceinline__ void uniform_step(const float (&v)[B][1 << K][NE], co
                 bits |= bf[j] << (K * j);
             }
             __builtin_memcpy(__builtin_assume_aligned(curr + (size_t)t * 2 * stride + blk * NE, NE * 2), h, NE * 2);
-            if (BACK) row[(size_t)t * back_tile + blk] = (BackWord<NE, K>)bits;
+            if (BACK) row[(size_t)t * back_tile + blk] = (uint8_t)bits;
         }
     }
 }
 
-// Up to 16 values a thread, two workgroups share a CU (at most 128 VGPRs): one's barriers under the other's steps.
+// Up to 16 values a thread are bound to the 128 VGPRs of two workgroups a CU, one's barriers under the other's steps (the
+// 32 values of K = 2 and 3 with two blocks fit them too).
 template <int FAM, int NE, int K, int B>
-__global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void encode_uniform_kernel(const float *__restrict__ tiles, int64_t count,
-                                                                     int T, int w, DecodeK dk,
-                                                                     uint16_t *__restrict__ packed,
-                                                                     double *__restrict__ sse,
-                                                                     float *__restrict__ recon,
-                                                                     uint8_t *__restrict__ back_ws) {
-    using Word = BackWord<NE, K>;
+__global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void encode_uniform_kernel(
+    const float *__restrict__ tiles, int64_t count, int T, int w, DecodeK dk, uint16_t *__restrict__ packed,
+    double *__restrict__ sse, float *__restrict__ recon, uint8_t *__restrict__ back_ws) {
+    static_assert(NE * K <= 8, "a block's backpointers are one byte");
     constexpr int KK = 1 << K;
     extern __shared__ __align__(16) unsigned char enc_lds[];
     const int kr = w - K, stride = 1 << kr, blocks = stride / NE;
@@ -329,8 +322,8 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
     uint32_t *red = words + T * 64;
     int *pin = reinterpret_cast<int *>(red + (ENC_THREADS / 64) * T);
 
-    const size_t back_tile = (size_t)256 * blocks;  // Words
-    Word *back = reinterpret_cast<Word *>(back_ws + (size_t)blockIdx.x * T * 256 * stride);
+    const size_t back_tile = (size_t)256 * blocks;
+    uint8_t *back = back_ws + (size_t)blockIdx.x * T * 256 * stride;
     const int64_t batches = (count + T - 1) / T;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int block = B == 1 ? tid & (blocks - 1) : tid;
@@ -347,13 +340,12 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
                 v[b][f][j] = __half2float(
                     decode1<FAM>(((uint32_t)f << kr) | (uint32_t)((block + b * ENC_THREADS) * NE + j), dk));
 
-    // Traceback geometry: half a wave per tile (T <= 16), rows of blocks * sizeof(Word) bytes, chunks of `rows` rows
-    // that fit the tile's cost rows.
+    // Traceback geometry: half a wave per tile (T <= 16), rows of `blocks` bytes, chunks of `rows` rows that fit the
+    // tile's cost rows (1024 bytes at the narrowest, n = 64 at 12 bits).
     const int ht = tid >> 5, hl = tid & 31;
-    const int row_bytes = blocks * (int)sizeof(Word);
     const int chunk = 4 * stride < CHUNK_BYTES ? 4 * stride : CHUNK_BYTES;
     // Rows wider than a chunk are walked in place.
-    const int rows = row_bytes <= chunk ? chunk / row_bytes : 0;
+    const int rows = blocks <= chunk ? chunk / blocks : 0;
 
     for (int64_t bt = blockIdx.x; bt < batches; bt += gridDim.x) {
         const int64_t tile0 = bt * T;
@@ -373,7 +365,7 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
                 const int ri = (step + roll) & 255;
                 const uint16_t *prev = costs + (step & 1) * stride;
                 uint16_t *curr = costs + ((step & 1) ^ 1) * stride;
-                Word *row = back + (size_t)ri * blocks;
+                uint8_t *row = back + (size_t)ri * blocks;
                 if (pass == 0 && step < 128)
                     uniform_step<NE, K, B, false>(v, xs, ri, T, set, sets, block, prev, curr, stride, pstep, row,
                                                   back_tile);
@@ -405,10 +397,10 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
             }
             // Traceback of trellis steps 127 .. 0 (pass 0) or 255 .. 0 (pass 1), whose rows lie in order of ri.
             if (ht < T) {
-                const Word *src = back + (size_t)ht * back_tile;
+                const uint8_t *src = back + (size_t)ht * back_tile;
                 const int top = pass == 0 ? 128 : 256;
                 int edge = pin[ht];
-                auto walk = [&](const Word *r, int ri) {
+                auto walk = [&](const uint8_t *r, int ri) {
                     const int fresh = ((uint32_t)r[edge / NE] >> (K * (edge & (NE - 1)))) & (KK - 1);
                     const int state = (fresh << kr) | edge;
                     edge = state >> K;
@@ -416,11 +408,12 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
                 };
                 if (rows != 0) {
                     unsigned char *stage = enc_lds + (size_t)ht * 4 * stride;
-                    const unsigned char *bytes = reinterpret_cast<const unsigned char *>(src);
                     uint4 q0, q1, q2, q3;  // a chunk's shares of this lane, 512 bytes apart
+                    // (`two` holds for every chunk there is, 1024 bytes at the least; without the condition the compiler
+                    // lays the kernel out another way and 4096 tiles at n = 32, w = 12 take 1204 us instead of 1195)
                     const bool two = chunk > 512, four = chunk > 1024;
                     auto fetch = [&](int c) {
-                        const unsigned char *from = bytes + (size_t)c * chunk + hl * 16;
+                        const uint8_t *from = src + (size_t)c * chunk + hl * 16;
                         q0 = *reinterpret_cast<const uint4 *>(from);
                         if (two) q1 = *reinterpret_cast<const uint4 *>(from + 512);
                         if (four) q2 = *reinterpret_cast<const uint4 *>(from + 1024);
@@ -440,7 +433,7 @@ __global__ __launch_bounds__(ENC_THREADS, (B * NE << K) <= 16 ? 4 : 2) void enco
                         __builtin_amdgcn_wave_barrier();
                         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                         for (int r = rows - 1; r >= 0; r--)
-                            walk(reinterpret_cast<const Word *>(stage + r * row_bytes), c * rows + r);
+                            walk(stage + r * blocks, c * rows + r);
                         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                         __builtin_amdgcn_wave_barrier();
                         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -476,7 +469,8 @@ hipError_t launch_uniform(const EncodeArgs &a, hipStream_t s) {
 template <int FAM, int K>
 hipError_t launch_uniform_k(const EncodeArgs &a, hipStream_t s) {
     constexpr int NE = K == 2 ? 4 : 2;
-    if (K < 4 && a.tiles_per_wg == 1 && a.w == 12) return launch_uniform<FAM, K == 2 ? 2 : 1, K, 1>(a, s);
+    if constexpr (K < 4)
+        if (a.tiles_per_wg == 1 && a.w == 12) return launch_uniform<FAM, K == 2 ? 2 : 1, K, 1>(a, s);
     switch (a.stride / NE / ENC_THREADS) {
     case 0:
     case 1: return launch_uniform<FAM, NE, K, 1>(a, s);
