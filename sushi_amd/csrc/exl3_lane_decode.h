@@ -106,9 +106,9 @@ struct CodewordOrder {
 struct OrderAll {  // all 32 in order
     static constexpr int at(int i) { return i; }
 };
-template <int N, int G>
-struct OrderGroup {  // group G of two, 16 codewords whose windows hold no other group's (8 apart for n = 16)
-    static constexpr int at(int i) { return N == 16 ? (i < 8 ? 8 * G + i : 8 + 8 * G + i) : 16 * G + i; }
+template <int G>
+struct OrderGroup {  // group G of two, 16 codewords
+    static constexpr int at(int i) { return 16 * G + i; }
 };
 template <int H, int G>
 struct OrderHalf {  // group G of two of the half decode: column j + 8 H, 8 codewords
@@ -116,9 +116,9 @@ struct OrderHalf {  // group G of two of the half decode: column j + 8 H, 8 code
 };
 
 // The weights of the lane's chunk, unscaled for the hash / pair families (the x4096 is applied by the caller).
-// GROUPED: the phases over two groups of 16 codewords, half the temporaries (a caller whose accumulators need the
-// registers); the others run all 32 together where the rate pairs its windows.
-template <int FAM, int N, bool MASKED, bool GROUPED = !Pairing<N>::ON>
+// The hash-product families run all 32 codewords together where the rate pairs its windows (two codewords each), else in
+// two groups of 16, half the temporaries.
+template <int FAM, int N, bool MASKED>
 __device__ __forceinline__ void decode_weights(const uint32_t (&A)[LaneBits<N>::AW], const DecodeK &k,
                                                uint32_t (&w)[16]) {
     using P = Pairing<N>;
@@ -169,14 +169,14 @@ __device__ __forceinline__ void decode_weights(const uint32_t (&A)[LaneBits<N>::
         });
     } else {
         const DecodeV v = decode_vgprs<FAM>(k);
-        if constexpr (!GROUPED) {
+        if constexpr (P::ON) {
             uint32_t c[32];
             lane_codewords<N, 32, MASKED>(A, v, c, CodewordOrder<N, 32, OrderAll>{});
             hash_weights<FAM, 32>(c, v, w);
         } else {
             unrolled<2>([&](auto gc) __attribute__((always_inline)) {
                 constexpr int g = decltype(gc)::value;
-                using O = OrderGroup<N, g>;
+                using O = OrderGroup<g>;
                 uint32_t c[16], p[8];
                 lane_codewords<N, 16, MASKED>(A, v, c, CodewordOrder<N, 16, O>{});
                 hash_weights<FAM, 16>(c, v, p);
@@ -213,7 +213,7 @@ __device__ __forceinline__ void decode_weights_half(const uint32_t (&A)[LaneBits
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Per-tile rates (configs[4]'s seeded K1 / K2 tile mix, a layout extension: the reference fixes a rate per tensor or
+// Per-tile rates (a seeded K1 / K2 tile mix, a layout extension: the reference fixes a rate per tensor or
 // per expert group, src/exl3/layout.zig:56-62, and decodes every tile at its own n with decodeTile,
 // src/exl3/expert_exl3.zig:338-357).  A segment is the 8 tiles (k-tile row tk, output group s) one wave reads; they
 // lie contiguous from the segment's word offset, tile o at TILED_NA halfwords when bit o of the segment's mask is set,
