@@ -1,5 +1,5 @@
-"""Headline benchmark: EXL3 K=4 4096x4096 decode GEMV at batch 1 (BASELINE.json configs[0]'s shape, run on the GPU)
-plus the MoE gathered-expert layer (configs[3], batch 1) as a secondary figure.
+"""Headline benchmark: EXL3 K=4 4096x4096 decode GEMV at batch 1 plus the MoE gathered-expert
+layer (256 experts + shared, 2048 x 768, K2, top-8; batch 1) as a secondary figure.
 
 A step is one call of the hot path (prepare + trellis-decode GEMV + finish) on one token of seeded synthetic fp16
 input.  Weights rotate over 64 resident copies (537 MB > the 256 MB Infinity Cache).  The calls are captured as HIP
@@ -10,7 +10,7 @@ timed call reads a copy last read 64 calls (537 MB of other weights) earlier: fr
 events around two graphs, the 64-copy sequence and the same sequence followed by the `--steps` timed calls: their
 difference is the timed calls back to back inside one graph, without the start cost of a second graph.
 
-Prints one JSON line (the driver's contract).  `cpu_baseline` times the C restatement of the reference's CPU path
+Prints one JSON line.  `cpu_baseline` times the C restatement of the reference's CPU path
 (oracle/, `expert_exl3.project`) on a bounded sample of the same workload, on every host core and on one.
 """
 from __future__ import annotations
@@ -146,7 +146,7 @@ def bench_linear(steps: int, warmup: int, graph_mode: bool = True, rounds: int =
 
 
 def bench_moe(batch: int, layers: int = 16, rounds: int = ROUNDS):
-    """E=256 routed + shared, hidden 2048, inter 768, K2 MCG, top-8; microseconds per token.
+    """The routed MoE layer: E=256 routed + shared, hidden 2048, inter 768, K2 MCG, top-8; microseconds per token.
 
     `layers` MoE layers back to back on one stream, captured once as a HIP graph and replayed: the stream runs them
     in order, as the reference's dependent chain (bench_util.zig:20-58) runs its calls, but each layer reads its own
@@ -479,7 +479,7 @@ def bench_pack(pair_major: bool, experts: int = 256, hidden: int = 2048, inter: 
 
 
 def sweep(which: str, prefill_batches=None, prefill_arms=("gemm", "windows"), c2_filter=None):
-    """configs[1] (C2: MCG GEMV sweep), configs[2] (C3: prefill GEMM) and configs[4] (C5: ragged STQ MoE layer):
+    """C2 (the MCG GEMV over shapes, rates and rows), C3 (the prefill GEMM) and C5 (the ragged STQ MoE layer):
     one JSON line per case."""
     from sushi_amd import exl3
 
@@ -562,7 +562,7 @@ def _graph_layer_us(chain, dev, layers: int, rounds: int = ROUNDS) -> float:
 
 
 def _c5_inputs(E: int, batch: int, layers: int, dev):
-    """configs[4]'s per-layer inputs: each layer its own N(0,1) hidden state and top-8 routing over N(0,1) logits."""
+    """C5's per-layer inputs: each layer its own N(0,1) hidden state and top-8 routing over N(0,1) logits."""
     import torch
 
     from sushi_amd import exl3, synth
@@ -585,7 +585,7 @@ def _c5_line(variant: str, batch: int, E: int, bpw: float, layer_us: float, alg:
 
 
 def bench_moe_c5(batch: int = 64, layers: int = 4):
-    """configs[4] in the reference-expressible form: the per-expert rate groups of rate_groups.zig (64 experts at
+    """C5 in the reference-expressible form: the per-expert rate groups of rate_groups.zig (64 experts at
     K=1, 192 at K=2: 1.75 bpw on average) as one ragged bank, hidden 4096, inter 2048, SPEC1 (spec1-w15 table: the
     one with K=1 rows), top-8 over N(0,1) logits, batch 64, plus a K=4 shared expert run as a one-expert chain whose
     output the routed call adds.  `layers` layers, each with its own input and routing, captured once; median of
@@ -623,7 +623,7 @@ def bench_moe_c5(batch: int = 64, layers: int = 4):
 
 
 def bench_moe_c5_tiled(batch: int = 64, layers: int = 4):
-    """configs[4] as stated: every expert's tiles at a seeded per-tile mix of K=1 and K=2 (25% K1; the realised rate is
+    """C5 with per-tile rates: every expert's tiles at a seeded per-tile mix of K=1 and K=2 (25% K1; the realised rate is
     reported), 256 experts, hidden 4096, inter 2048, SPEC1 (spec1-w15), top-8 over N(0,1) logits, batch 64, plus a
     K=4 shared expert -- in the same launches (moe_tiled_with_shared_bank, "tiled_fused") and as the pair of calls
     (one-expert chain, then moe_tiled with its output, "tiled_pair").  Bytes: the distinct experts' packed tiles,
@@ -673,7 +673,7 @@ def bench_moe_c5_tiled(batch: int = 64, layers: int = 4):
 
 
 def bench_moe_prefill(batches=(64, 128, 256, 512, 1024, 2048), layers: int = 4, arms=("gemm", "windows")):
-    """configs[3]'s layer (E=256 + shared, hidden 2048, inter 768, K2 MCG, top-8) at prefill widths, on the routed
+    """The routed MoE layer (E=256 + shared, hidden 2048, inter 768, K2 MCG, top-8) at prefill widths, on the routed
     GEMM arm and on the decode chain's expert windows (arm overrides): microseconds per layer and per token, each a
     median of 7 replays of `layers` layers from a HIP graph."""
     import statistics
@@ -724,7 +724,7 @@ def bench_moe_prefill(batches=(64, 128, 256, 512, 1024, 2048), layers: int = 4, 
 
 def bench_moe_prefill_c5(batches=(256, 512, 1024, 2048), layers: int = 2, arms=("gemm", "windows"),
                          forms=("ragged", "tiled")):
-    """configs[4]'s layer (hidden 4096, inter 2048, 256 experts at 1.75 bpw, SPEC1 spec1-w15, top-8, plus a K=4 shared
+    """C5's layer (hidden 4096, inter 2048, 256 experts at 1.75 bpw, SPEC1 spec1-w15, top-8, plus a K=4 shared
     expert) at prefill widths, on the routed GEMM arm and on the GEMV expert windows (arm overrides), for the ragged
     rate-group bank (64 experts at K1, 192 at K2) and the per-tile K1 / K2 bank; the shared expert rides the routed
     launches where the fused form serves, else runs as the pair of calls.  Median of 7 replays of `layers` layers
@@ -871,7 +871,7 @@ def cpu_baseline(sample_calls: int):
 
 
 def cpu_moe_baseline(batch: int = 16):
-    """moeSwigluHost (expert_exl3_kernels.zig:3059-3114) over configs[3]'s layer: 256 experts, hidden 2048, inter 768,
+    """moeSwigluHost (expert_exl3_kernels.zig:3059-3114) over the routed MoE layer: 256 experts, hidden 2048, inter 768,
     K2 MCG, top-8 over N(0,1) logits plus the shared expert as a ninth slot of weight 1; us per token on every core
     (OpenMP over `batch` rows) and on one (a single token); median of 7 samples."""
     import statistics
@@ -927,10 +927,10 @@ def main() -> int:
     ap.add_argument("--no-twin", action="store_true", help="skip the MCG twin of the headline GEMV")
     ap.add_argument("--no-ceilings", action="store_true", help="skip the measured read/copy/8 MiB-launch ceilings")
     ap.add_argument("--no-graph", action="store_true", help="issue every call from Python instead of a HIP graph")
-    ap.add_argument("--moe-batches", default="1,8,32", help="MoE layer batches (configs[3]); the first is headline")
+    ap.add_argument("--moe-batches", default="1,8,32", help="MoE layer batches; the first is headline")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
                     help="first copy MIB MiB device-to-device 4 times (the counter-calibration kernel)")
-    ap.add_argument("--sweep", choices=("c2", "c3", "c5", "moe_prefill", "c5_prefill", "enc", "pack", "all"), help="time configs[1]/[2] cases instead (one JSON line each)")
+    ap.add_argument("--sweep", choices=("c2", "c3", "c5", "moe_prefill", "c5_prefill", "enc", "pack", "all"), help="time these cases instead (one JSON line each)")
     ap.add_argument("--prefill-batches", default="", help="moe_prefill sweep: token counts (default 64 .. 2048)")
     ap.add_argument("--prefill-arms", default="gemm,windows", help="moe_prefill sweep: arms to time")
     ap.add_argument("--c2-cases", default="", help="c2 sweep: only these cases, e.g. 2048x2048:32:1,2048x2048:32:16 "

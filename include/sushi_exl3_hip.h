@@ -117,7 +117,7 @@ typedef struct {
     int32_t lane_rates_only;
 } exl3_ragged_t;
 
-/* A per-tile-rate bank (configs[4]'s seeded K1 / K2 tile mix).  No counterpart in the reference, which fixes a rate
+/* A per-tile-rate bank (a seeded K1 / K2 tile mix).  No counterpart in the reference, which fixes a rate
  * per tensor (src/exl3/layout.zig:56-62) or per expert group (src/exl3/rate_groups.zig:22-140); each tile still
  * decodes at its own n as decodeTile does (src/exl3/expert_exl3.zig:338-357), so this is a layout extension.  A
  * segment is the 8 tiles (k-tile row tk, output tiles 8s .. 8s + 7) of one expert's projection: segment index

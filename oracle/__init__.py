@@ -338,7 +338,7 @@ def moe_swiglu_rows(x, gate, up, down, slots, weights, hidden: int, inter: int, 
     return y
 
 
-# ---- per-tile rates (configs[4]'s K1/K2 tile mix; an extension with no reference counterpart) ----------------
+# ---- per-tile rates (a K1/K2 tile mix; an extension with no reference counterpart) -------------------------
 
 
 def reconstruct_inner_tiled(trellis, seg_off, seg_k1, expert: int, in_f: int, out_f: int, n_a: int, n_b: int,

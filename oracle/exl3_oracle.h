@@ -28,7 +28,7 @@
  *                                   independent numpy restatement over ox_decode_dense weights.
  *   ox_moe_swiglu_rows            : rows of ox_moe_swiglu_host over ragged banks; equals it row by row (and the
  *                                   threaded run equals the single-threaded one byte for byte).
- *   ox_*_tiled                    : EXTENSION (configs[4]'s per-tile K1/K2 map, no reference counterpart): the
+ *   ox_*_tiled                    : EXTENSION (a per-tile K1/K2 map, no reference counterpart): the
  *                                   uniform functions applied tile by tile at each tile's own rate; equal to them
  *                                   when every tile has one rate, and to per-tile decodeTile reassembly otherwise.
  *   ox_gated_shared_term          : the rounding chain of REDUCE_GATED_SHARED_SOURCE; checked against numpy's

@@ -1,7 +1,7 @@
 """Builds libsushi_exl3_hip.so in-tree with hipcc for gfx950 (one object per translation unit, in parallel).
 
-Run as ``python -m sushi_amd.build`` or through ``__graft_entry__.build()``.  Every call recompiles (the driver's
-"does it build" check); ``load()`` in ``sushi_amd._lib`` only loads what is built.
+Run as ``python -m sushi_amd.build`` or through ``__graft_entry__.build()``.  Every call recompiles;
+``load()`` in ``sushi_amd._lib`` only loads what is built.
 """
 from __future__ import annotations
 

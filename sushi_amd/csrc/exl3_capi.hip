@@ -60,8 +60,14 @@ constexpr int kMaxDevices = 64;  // devices with per-device state (the no-alloc 
 
 bool rate_admitted(int n) { return n >= 16 && n <= 128 && n % 2 == 0; }  // kFromPackedDim, expert_exl3.zig:241-245
 
-// The rates the GEMV and the GEMM read with a lane reader.
+// The rates that every kernel reads with a lane reader: the routed GEMM arm, the fused chain, fused shared experts and
+// rate-grouped banks take these alone.
 bool lane_rate(int n) { return n == 16 || n == 24 || n == 32 || n == 40 || n == 48 || n == 64; }
+
+// The rates that the GEMV (dense, and a uniform bank's slots and windows) and the dense GEMM read with one: K = 5 .. 8
+// too, as launch_gemv_fam and launch_gemm_fam switch them.  Any other rate takes the generic reader, and its dense GEMM
+// a transposed f16 copy in the workspace.
+bool dense_lane_rate(int n) { return lane_rate(n) || n == 80 || n == 96 || n == 112 || n == 128; }
 
 // Arm overrides (exl3_set_override): one word per knob, INT32_MIN = unset.  Read with a relaxed load at each call,
 // so an unset knob costs one load and nothing in the environment changes an arm.
@@ -183,8 +189,7 @@ uint32_t gemm_split_wait(long workgroups) {
 
 size_t gemm_bytes(int groups, int rows, int in, int out, int n, bool split_ok = true) {
     size_t b = kZeroBytes + gemm_xp_bytes(groups, rows, in);
-    const bool lane_reader = lane_rate(n) || n == 80 || n == 96 || n == 112 || n == 128;
-    if (!lane_reader) b += align_up((size_t)groups * out * in * 2);  // the transposed f16 copy of other rates
+    if (!dense_lane_rate(n)) b += align_up((size_t)groups * out * in * 2);  // the transposed f16 copy
     if (gemm_uses_kpart(groups, rows, out, n, split_ok)) b += align_up(gemm_kpart_bytes(groups, rows, out));
     return b;
 }

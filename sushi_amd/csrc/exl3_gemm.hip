@@ -264,7 +264,7 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_kernel(GemmArgs a, const uint
     }
 }
 
-// ---- the decode-once GEMM (integer and half-integer rates with a lane reader: n = 16, 24, 32, 40, 48, 64)
+// ---- the decode-once GEMM (integer and half-integer rates with a lane reader: n = 16, 24, 32, 40, 48, 64, 80, 96, 112, 128)
 //
 // A workgroup owns a 256-row x 128-column output tile (one Hadamard block wide, so the FWHT + svh finish runs in its
 // epilogue) over all of k, in super-steps of 128 k (eight trellis k-tile rows), with the decode and the MFMAs on
@@ -374,7 +374,7 @@ struct RateReader {
     }
 };
 
-// A per-tile-rate projection (configs[4]'s K1 / K2 mix): the row of load i is segment seg0 + i * seg_step, at the
+// A per-tile-rate projection (a K1 / K2 mix): the row of load i is segment seg0 + i * seg_step, at the
 // word offset and with the rate mask of the segment tables; lane 8 o + j's tile starts 16 o - 8 popcount(mask below o)
 // words in, at TILED_NA when bit o is set.  The segment's offset and mask (scalar loads) are fetched two loads ahead,
 // so a tile's vector loads never wait on them, also where a decoder issues two loads back to back.
@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mid_kernel(MoeGemmArgs a) {
 
 template <int DT>
 static void launch_moe_gemm_prepare(const MoeGemmArgs &a, hipStream_t s) {
-    // two 128-column blocks a workgroup where they pair up (measured at 2048 tokens of configs[3]: 85 -> 79 us; four
+    // two 128-column blocks a workgroup where they pair up (measured at 2048 tokens of 2048 x 768, top-8 of 256: 85 -> 79 us; four
     // blocks took 110)
     const int blocks = a.in / 128;
     if (blocks % 2 == 0)

@@ -1085,7 +1085,7 @@ static hipError_t launch_gemv_fam(const GemvArgs &a, hipStream_t s) {
     }
     // K = 5 .. 8 of a uniform bank (PAIR1 has no rows there): the lane reader reads each lane's words once and funnels
     // at fixed positions, where the generic reader finds every codeword's word pair at run time.  One row through
-    // 5120 x 129280 at n = 96 (SPEC1, f32 out): 915 us on the generic reader, 151 us here.
+    // 5120 x 129280 at n = 96 (SPEC1, f32 out): 915 us on the generic reader, 138 us here.
     if constexpr (FAM != FAM_PAIR) {
         switch (a.n) {
         case 80: return launch_gemv_n<FAM, 80, PRO>(a, s);

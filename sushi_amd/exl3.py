@@ -259,7 +259,8 @@ class Bank:
 
 META_WORDS = 8
 
-# Rates the kernels read with a per-lane fixed-width reader; any other rate takes the generic reader.
+# Rates that a rate-grouped bank's kernels read with a per-lane fixed-width reader; its experts of any other rate take the
+# generic reader.  (Dense weights and uniform banks have lane readers at n = 80, 96, 112 and 128 as well.)
 LANE_RATES = (16, 24, 32, 40, 48, 64)
 
 
@@ -338,7 +339,7 @@ def _as_i32(t: torch.Tensor) -> torch.Tensor:
 
 @dataclass
 class TiledProj:
-    """One projection of a per-tile-rate bank (configs[4]'s K1 / K2 tile mix), a layout extension: the reference fixes
+    """One projection of a per-tile-rate bank (a K1 / K2 tile mix), a layout extension: the reference fixes
     a rate per tensor (layout.zig:56-62) or per expert group (rate_groups.zig:22-140), while each tile's arithmetic is
     decodeTile's at that tile's own n (expert_exl3.zig:338-357).
 

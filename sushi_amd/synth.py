@@ -8,7 +8,7 @@ same bytes.
   codes  : uniform u16, 4 per 64-bit draw (little-endian halfwords)
   suh/svh: sign (+-1, from bit 63) x U(0.5, 1.5), rounded to f16
   x      : N(0, 1) by Box-Muller over two uniform draws, rounded to f16
-  k1 map : a tile is K1 where its U[0, 1) draw is below p_k1 (configs[4]: 0.25), else K2
+  k1 map : a tile is K1 where its U[0, 1) draw is below p_k1 (0.25 unless named), else K2
 """
 from __future__ import annotations
 
@@ -109,7 +109,7 @@ def bank(seed: int, name: str, experts: int, hidden: int, inter: int, n, device=
 
 
 def tile_map(seed: int, name: str, shape, p_k1: float = 0.25, device="cpu") -> torch.Tensor:
-    """configs[4]'s seeded per-tile rate map: each tile K1 (True) with probability p_k1, else K2."""
+    """A seeded per-tile rate map: each tile K1 (True) with probability p_k1, else K2."""
     return (uniform01(seed_of(seed, name), math.prod(shape)) < p_k1).reshape(shape).to(device)
 
 

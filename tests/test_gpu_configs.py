@@ -1,7 +1,7 @@
-"""The routed configurations at their full shapes against the oracle (max-abs-rel 2e-3, BASELINE.json north_star).
+"""The routed configurations at their full shapes against the oracle (max-abs-rel 2e-3).
 
-configs[3] (C4): 256 routed experts + 1 shared, hidden 2048, inter 768, K2 MCG, top-8 over N(0,1) logits, batch 1 / 8 /
-32 -- the shapes bench.py times, through the same calls (moe_with_shared_bank; and moe alone).  configs[4] (C5) in the
+C4: 256 routed experts + 1 shared, hidden 2048, inter 768, K2 MCG, top-8 over N(0,1) logits, batch 1 / 8 /
+32 -- the shapes bench.py times, through the same calls (moe_with_shared_bank; and moe alone).  C5 in the
 reference's rate-group form: 64 experts at K1 and 192 at K2 (1.75 bpw), SPEC1 with the spec1-w15 table, hidden 4096,
 inter 2048, top-8, batch 64 on the sorted arm, plus a K4 shared expert; and as stated, a seeded per-tile K1 / K2 mix in
 every expert (exl3.Tiled).  The oracle is moeSwigluHost
@@ -71,7 +71,7 @@ def test_c4_layer_with_shared_expert(dev, c4, batch):
 
 
 def test_c5_rate_group_layer_batch_64(dev):
-    """configs[4] in the rate-group form: SPEC1 K1/K2 experts (a ragged bank), K4 shared expert, batch 64."""
+    """C5 in the rate-group form: SPEC1 K1/K2 experts (a ragged bank), K4 shared expert, batch 64."""
     print("[c5] batch=64", flush=True)
     E1, E2, hidden, inter, k, batch = 64, 192, 4096, 2048, 8, 64
     dec, odec = exl3.Decode(exl3.Codebook.spec1, exl3.Window(15), 1), O.decode(O.CB_SPEC1, 15, 1)
@@ -100,7 +100,7 @@ def test_c5_rate_group_layer_batch_64(dev):
 
 
 def test_c5_per_tile_layer_batch_64(dev):
-    """configs[4] as stated: every expert at a seeded per-tile K1 / K2 mix (25 % K1), SPEC1 (spec1-w15), hidden 4096,
+    """C5 with per-tile rates: every expert at a seeded per-tile K1 / K2 mix (25 % K1), SPEC1 (spec1-w15), hidden 4096,
     inter 2048, top-8 over 256 experts, batch 64 on the sorted arm, with a K4 shared expert in the same launches."""
     print("[c5] per-tile batch=64", flush=True)
     E, hidden, inter, k, batch = 256, 4096, 2048, 8, 64
@@ -126,7 +126,7 @@ def test_c5_per_tile_layer_batch_64(dev):
 
 
 def test_c4_prefill_width_takes_the_gemm_arm(dev, c4):
-    """configs[3]'s layer at a 512-token prefill (4096 slots, 16 per expert on average): the routed GEMM arm (taken
+    """C4's layer at a 512-token prefill (4096 slots, 16 per expert on average): the routed GEMM arm (taken
     by itself at this width) against the oracle, and equal to the decode chain at the bar."""
     print("[c4] prefill 512", flush=True)
     b, sh, bd, shd, banks = c4

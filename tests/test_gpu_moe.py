@@ -145,7 +145,7 @@ def test_moe_ragged_lane_flag_clear_is_correct(dev, monkeypatch):
 
 
 def test_moe_ragged_stq_rates_k1_k2(dev):
-    """configs[4]'s layer in its reference-expressible form: per-expert rate groups at K=1 and K=2 (1:3), SPEC1
+    """The rate-grouped layer in its reference-expressible form: per-expert rate groups at K=1 and K=2 (1:3), SPEC1
     with the spec1-w15 table (the SPEC1 table with K=1 rows), plus a shared expert, against the oracle."""
     hidden, inter, k, rows = 256, 128, 8, 5
     groups = [(4, (16, 16, 16)), (12, (32, 32, 32))]

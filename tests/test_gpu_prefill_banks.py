@@ -8,7 +8,7 @@ banks) while the MFMA waves are the uniform arm's.  Checked:
   * against the oracle (moeSwigluHost over every row, max-abs-rel 2e-3) for the codebooks and rates each form admits,
     with and without a clamp and a (gated) shared expert;
   * a fused shared bank in the same launches equals the reference callers' pair of calls bit for bit;
-  * configs[4]'s layer (hidden 4096, inter 2048, 1.75 bpw, SPEC1 spec1-w15) at 1024 tokens on the summand-relative bar
+  * C5's layer (hidden 4096, inter 2048, 1.75 bpw, SPEC1 spec1-w15) at 1024 tokens on the summand-relative bar
     (tests/_parity.py), with the reference's mutation arms: the wrong codeword window and one flipped trellis bit must
     fail it (src/exl3/expert_exl3_kernels.zig:3310-3352).
 """
@@ -168,7 +168,7 @@ def test_shared_bank_rides_the_gemm_arm_of_ragged_and_tiled_banks(dev, form, dty
     assert torch.equal(y, ref)
 
 
-# ---- configs[4]'s layer at a 1024-token prefill on the summand-relative bar ----------------------------------------
+# ---- C5's layer at a 1024-token prefill on the summand-relative bar ------------------------------------------------
 #
 # Each token routes all 8 of its slots to one expert (scores summing to 1), so y = svh_down[e] * H(inner_down) of that
 # expert is undone exactly (tests/test_gpu_parity.py routes the same way); 1024 tokens over 16 experts, half of them

@@ -1,4 +1,4 @@
-"""Per-tile-rate banks (configs[4]'s seeded K1 / K2 tile mix) on the GPU, against the oracle's per-tile functions.
+"""Per-tile-rate banks (a seeded K1 / K2 tile mix) on the GPU, against the oracle's per-tile functions.
 
   * exl3_reconstruct_tiled -- the routed GEMV's tiled reader and decoder -- is bit-exact with
     reconstruct_inner_tiled (each tile through decodeTile at its own rate, src/exl3/expert_exl3.zig:338-357) for the

@@ -1,4 +1,4 @@
-"""Pins the oracle's per-tile-rate functions (configs[4]'s K1 / K2 tile mix, a layout extension with no reference
+"""Pins the oracle's per-tile-rate functions (a seeded K1 / K2 tile mix, a layout extension with no reference
 counterpart) and the host packer that lays such a bank out (exl3.TiledProj.pack).
 
 The tile arithmetic is decodeTile's at each tile's own rate (src/exl3/expert_exl3.zig:338-357), which the golden
