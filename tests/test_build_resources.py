@@ -1,6 +1,6 @@
 """Every kernel of the built gfx950 library runs without scratch memory and without VGPR spills, the PAIR decode GEMV
-keeps the registers of three workgroups a CU, and no matrix instruction reads a VGPR that a vector instruction wrote
-fewer than three instructions before it.
+keeps the registers of three workgroups a CU, the uniform encoder search keeps those its plan counts on, and no matrix
+instruction reads a VGPR that a vector instruction wrote fewer than three instructions before it.
 
 Read from the code-object metadata of the objects `python -m sushi_amd.build` leaves in sushi_amd/_build
 (`.private_segment_fixed_size`, `.vgpr_spill_count`).  Scratch in these kernels has meant the compiler copying a
@@ -82,6 +82,21 @@ def test_pair_gemv_keeps_three_workgroups_a_cu(tmp_path):
     assert len(vgprs) == 18, sorted(vgprs)
     over = {n: v for n, v in vgprs.items() if v > 80}
     assert not over, over
+
+
+@pytest.mark.skipif(not OBJECTS or not (os.path.exists(BUNDLER) and os.path.exists(READELF) and shutil.which("objcopy")),
+                    reason="needs the built objects (python -m sushi_amd.build) and the ROCm binutils")
+def test_uniform_search_registers_are_what_its_plan_counts_on(tmp_path):
+    """encode_uniform_kernel<FAM, NE, K, B>: two workgroups of 512 threads a CU (at most 128 VGPRs) at K = 2 and 3 with up
+    to two blocks a thread (windows up to 14 bits), one for every other instance."""
+    seen = 0
+    for name, _, _, v in _kernels(os.path.join(BUILD, "exl3_encode.o"), str(tmp_path)):
+        m = re.search(r"encode_uniform_kernelILi\dELi\dELi(\d)ELi(\d)E", name)
+        if m:
+            seen += 1
+            two = int(m.group(1)) < 4 and int(m.group(2)) <= 2
+            assert (v <= 128) == two, (name, v)
+    assert seen == 39  # 13 shapes, 3 codebooks
 
 
 _VREG = re.compile(r"v\[(\d+):(\d+)\]|\bv(\d+)\b")

@@ -80,9 +80,9 @@ def test_gemv_codebooks_rates_rows(dev, label, n, rows):
 
 
 @pytest.mark.parametrize("n,label", [(16, "spec1"), (24, "pair1"), (40, "3inst"), (22, "spec1"), (44, "pair1"),
-                                     (96, "spec1"), (128, "spec1")])
+                                     (96, "spec1"), (128, "spec1"), (72, "spec1"), (90, "mcg"), (126, "mul1")])
 def test_gemv_other_rates(dev, n, label):
-    """n = 16, 24, 40 on the lane reader; 22, 44, 96, 128 on the generic reader."""
+    """n = 16, 24, 40, 96, 128 on the lane reader; 22, 44, 72, 90, 126 on the generic reader."""
     d = Dense(dev, 400 + n, 3, 256, 256, n)
     dec, odec = DECODES[label]
     _hold(d.inner(dec), d, odec, seed=n, what=f"gemv {label} n={n}")
@@ -100,7 +100,7 @@ def test_gemv_split_arms(dev, splits, separate):
 
 @pytest.mark.parametrize("seed", range(P.PARITY_SEEDS))
 def test_c1_headline_shape_every_seed(dev, seed):
-    """configs[0]'s shape as bench.py runs it: 4096 x 4096, K4 (n64), 3INST, batch 1."""
+    """The headline shape as bench.py runs it: 4096 x 4096, K4 (n64), 3INST, batch 1."""
     d = Dense(dev, seed, 1, 4096, 4096, 64)
     dec, odec = DECODES["3inst"]
     _hold(d.inner(dec), d, odec, seed=seed, what=f"c1 seed {seed}")
@@ -148,7 +148,7 @@ def _within_one_ulp(got: np.ndarray, y: np.ndarray, allow: np.ndarray):
 
 @pytest.mark.parametrize("label,seed", [("3inst", s) for s in range(P.PARITY_SEEDS)] + [("mcg", 0), ("mcg", 1)])
 def test_c1_fold_arm_every_output_within_one_f16_ulp(dev, label, seed):
-    """The arm bench.py times: configs[0]'s 4096 x 4096 K4 at batch 1 with an f16 output, which takes the fixed-point
+    """The arm bench.py times: 4096 x 4096 K4 at batch 1 with an f16 output, which takes the fixed-point
     fold over 8 splits (f32 outputs take the counters + planes arm, so the summand bar above never reaches it).  Every
     f16 output must sit within one f16 ulp of round_f16 of the f64 truth built from the oracle's decoded weights
     (src/exl3/expert_exl3_kernels.zig:3300-3352's standard, held per element; the allowance is a small fraction of an
@@ -185,7 +185,7 @@ def test_c1_fold_arm_every_output_within_one_f16_ulp(dev, label, seed):
 @pytest.mark.parametrize("n", [32, 48, 64])
 @pytest.mark.parametrize("in_f,out_f", [(2048, 2048), (4096, 14336), (14336, 4096)])
 def test_c2_shapes(dev, in_f, out_f, n, rows):
-    """configs[1] at full size: MCG, K = 2/3/4, batch 1/4/16."""
+    """The GEMV's shapes at full size: MCG, K = 2/3/4, batch 1/4/16."""
     d = Dense(dev, 1, rows, in_f, out_f, n)
     dec, odec = DECODES["mcg"]
     _hold(d.inner(dec), d, odec, seed=rows, mutate=in_f == out_f, what=f"c2 {in_f}x{out_f} n={n} rows={rows}")
@@ -200,6 +200,15 @@ def test_gemm_rates_rows(dev, n, rows):
     d = Dense(dev, 500 + rows, rows, 1024, 512, n)
     dec, odec = DECODES["3inst"]
     _hold(d.inner(dec), d, odec, seed=rows, what=f"gemm n={n} rows={rows}")
+
+
+@pytest.mark.parametrize("n,rows,label", [(22, 40, "spec1"), (36, 17, "3inst"), (44, 130, "pair1"), (72, 300, "spec1"),
+                                          (90, 33, "mcg"), (126, 130, "mul1")])
+def test_gemm_other_rates(dev, n, rows, label):
+    """The rates without a lane reader: decoded to a transposed f16 copy, then the 128-row tile."""
+    d = Dense(dev, 560 + n, rows, 384, 256, n)
+    dec, odec = DECODES[label]
+    _hold(d.inner(dec), d, odec, seed=n, what=f"gemm {label} n={n} rows={rows}")
 
 
 @pytest.mark.parametrize("rows", [40, 300])
@@ -227,7 +236,7 @@ def test_gemm_every_seed(dev, seed):
 
 @pytest.mark.parametrize("rows,out_f", [(512, 14336), (2048, 1024), (2048, 14336)])
 def test_c3_prefill_shapes(dev, rows, out_f):
-    """4096 x 14336, K3, 3INST at M = 512 (row tiles 2: the XCD remap with 4 output groups per XCD
+    """The prefill GEMM: 4096 x 14336, K3, 3INST at M = 512 (row tiles 2: the XCD remap with 4 output groups per XCD
     round) and M = 2048 (row tiles 8: one output group per XCD round), and M = 2048 at out 1024 (the same branch on a
     grid of one round)."""
     d = Dense(dev, 3, rows, 4096, out_f, 48)
