@@ -109,10 +109,10 @@ __device__ __forceinline__ uint32_t decode_pair_h2(uint32_t c0, uint32_t c1, con
 // ------------------------------------------------------------------------------------------------------------
 // Hand-scheduled gfx950 decode primitives for the GEMV's and GEMMs' hot loops.  What an instruction costs a SIMD with
 // four waves on it (cycles per wave64 instruction, independent destinations, the slowest wave timed): VGPR-only VOP1 /
-// VOP2 (and, add, shift, f16 add) 2.3-2.5 and v_bitop3 2.7, but 4.2 for the same with one SGPR operand; SDWA and the
-// other VOP3 (alignbit, bfe, mad_u32_u16, perm, packed) 4.2-4.4; v_mul_lo_u32 4.27, no more than its 16-bit parts;
-// v_mad_u16 with op_sel 8.3.  So the hash is one 32-bit product of the clean codeword (and / shift 2.4 + 4.27, where
-// two 16-bit steps took 8.5, 12.6 for the LCG), and every constant a step reads per weight sits in a VGPR.
+// VOP2 (and, add, shift, f16 add) 2.3 and v_bitop3 on three VGPRs 2.4, but 4.2 for the same with one SGPR operand; SDWA
+// and the other VOP3 (alignbit, bfe, mad_u32_u16, perm, packed) 4.4; v_mul_lo_u32 4.4, no more than its 16-bit parts;
+// v_mad_u16 with op_sel 8.2.  So the hash is one 32-bit product of the clean codeword (and / shift 2.3 + 4.4, where two
+// 16-bit steps took 8.7, 12.6 for the LCG), and every constant a step reads per weight sits in a VGPR.
 constexpr uint32_t LCG_A = 89226354u, LCG_B = 64248484u;
 
 // s in a VGPR that stays one: written in asm, so the compiler neither folds a scalar operand back in nor rebuilds the
